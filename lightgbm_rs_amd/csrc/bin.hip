@@ -120,7 +120,7 @@ __global__ __launch_bounds__(256) void k_bin_wide(const T* __restrict__ x, int64
   __shared__ DevBinFeature s_f[BIN_WIDE_F];
   __shared__ int32_t s_lo, s_hi;
   const int f0 = (int)blockIdx.y * BIN_WIDE_F;
-  const int nf = min(BIN_WIDE_F, F - f0);
+  const int nf = max(0, min(BIN_WIDE_F, F - f0));  // 0 in the words past the last feature
   if (threadIdx.x < (unsigned)nf) s_f[threadIdx.x] = feats[f0 + threadIdx.x];
   __syncthreads();
   if (threadIdx.x == 0) {
