@@ -30,6 +30,15 @@ void launch_predict(const PredNode* nodes, const PredTree* trees, const double* 
                     double es_margin, int32_t* es_iters, double* out, int32_t* leaf_out,
                     hipStream_t s, const KernelEvents* ev);
 int64_t shap_bytes_per_row(int32_t depth);
+int32_t shap_rows_per_block(int32_t nf, int32_t max_leaves);
+void launch_shap_paths(const PredNode* nodes, const PredTree* trees, const double* leaf_values,
+                       const int32_t* cat_bounds, const uint32_t* cat_words,
+                       const double* node_cover, const double* leaf_cover, const double* expected,
+                       const ShapLeaf* leaves, const ShapStep* steps, const int32_t* feats,
+                       const ShapPlan* plan, int64_t max_items, const float* X, int64_t rows,
+                       int32_t cols, int32_t nf, int32_t max_leaves, int32_t t0, int32_t t1,
+                       int32_t leaf0, int32_t leaf1, int32_t ntpi, int first, double* tab,
+                       double* out, hipStream_t s);
 void launch_csr_dense(const int64_t* indptr, const int32_t* indices, const float* values,
                       int64_t nnz, int64_t rows, int32_t cols, int32_t width, float* dense,
                       uint32_t* err, hipStream_t s);
@@ -142,6 +151,14 @@ struct lgbm_hip_ctx {
   size_t pm_csr_cap = 0;
   char* pm_shap = nullptr;  // TreeSHAP path workspace
   size_t pm_shap_cap = 0;
+  // the leaf paths of the model of pm_paths_uid (made when contributions are first asked
+  // of it), their depths and lengths on the host, and the last call's plan
+  uint64_t pm_paths_uid = 0;
+  ShapLeaf* pm_sleaf = nullptr;
+  ShapStep* pm_sstep = nullptr;
+  int32_t* pm_sfeat = nullptr;
+  ShapPlan* pm_splan = nullptr;
+  std::vector<int32_t> shap_dm;
   float* pm_x = nullptr;  // host-input staging
   size_t pm_x_cap = 0;
   void* pm_out = nullptr;
@@ -1465,6 +1482,10 @@ int lgbm_hip_ctx_destroy(lgbm_hip_ctx* c) {
   F(c->pm_lcov);
   F(c->pm_expv);
   F(c->pm_shap);
+  F(c->pm_sleaf);
+  F(c->pm_sstep);
+  F(c->pm_sfeat);
+  F(c->pm_splan);
   F(c->pm_csr);
   F(c->pm_x);
   F(c->pm_out);
@@ -3326,16 +3347,109 @@ int predict_prepare(lgbm_hip_ctx* c, const lgbm_hip_model* m, int64_t rows, int3
   return LGBM_HIP_OK;
 }
 
+// Feature contributions of iterations [it0, it1) by leaf paths (k_shap_items): the trees
+// in runs, and the rows in chunks where a tree needs it, whose values stay within 256 MiB.
+int contrib_paths(lgbm_hip_ctx* c, const lgbm_hip_model* m, const float* d_x, int64_t rows,
+                  int32_t cols, int32_t it0, int32_t it1, int32_t max_leaves, double* d_out) {
+  int rc = 0;
+  const int32_t ntpi = m->num_tree_per_iteration, nf = m->max_feature_idx + 1;
+  const int32_t nt0 = it0 * ntpi, nt1 = it1 * ntpi;
+  const size_t nleaf = m->leaf_values.size();
+  if (c->pm_paths_uid != m->uid) {
+    c->pm_paths_uid = 0;
+    ShapPaths p;
+    model_shap_paths(*m, &p);
+    if ((rc = upload_vec(c, &c->pm_sleaf, p.leaves))) return rc;
+    if ((rc = upload_vec(c, &c->pm_sstep, p.steps))) return rc;
+    if ((rc = upload_vec(c, &c->pm_sfeat, p.feats))) return rc;
+    if ((rc = dalloc(c, &c->pm_splan, nleaf))) return rc;
+    c->shap_dm.resize(nleaf);
+    for (size_t l = 0; l < nleaf; ++l) c->shap_dm[l] = p.leaves[l].dm;
+    c->pm_paths_uid = m->uid;
+  }
+  // values of a tree whose launch covers R rows: a leaf's items are the outcomes of its
+  // ancestors, or the rows where they are no more
+  auto items_of = [&](size_t leaf, int64_t R) {
+    const int32_t depth = c->shap_dm[leaf] & 0xffff;
+    return depth == 0 ? (int64_t)0 : std::min(R, (int64_t)1 << depth);
+  };
+  auto tree_values = [&](int32_t t, int64_t R) {
+    const PredTree& T = m->tree_index[(size_t)t];
+    int64_t v = 0;
+    for (int32_t l = 0; l < T.num_leaves; ++l)
+      v += items_of((size_t)T.leaf0 + l, R) * (c->shap_dm[(size_t)T.leaf0 + l] >> 16);
+    return v;
+  };
+  const int64_t most = ((int64_t)256 << 20) / 8;
+  int64_t chunk = rows, largest = 0;
+  for (int32_t t = nt0; t < nt1; ++t)
+    while (tree_values(t, chunk) > most) chunk = (chunk + 1) / 2;
+  struct Run {
+    int32_t t0, t1;
+    int64_t items;
+  };
+  std::vector<Run> runs;
+  std::vector<ShapPlan> plan(nleaf);
+  int64_t used = 0;
+  for (int32_t t = nt0; t < nt1; ++t) {
+    const PredTree& T = m->tree_index[(size_t)t];
+    const int64_t v = tree_values(t, chunk);
+    if (runs.empty() || used + v > most) {
+      runs.push_back({t, t, 0});
+      used = 0;
+    }
+    for (int32_t l = 0; l < T.num_leaves; ++l) {
+      const size_t leaf = (size_t)T.leaf0 + l;
+      const int64_t items = items_of(leaf, chunk);
+      const bool by_row = items > 0 && items < ((int64_t)1 << (c->shap_dm[leaf] & 0xffff));
+      plan[leaf] = ShapPlan{(uint32_t)used, (uint32_t)items | (by_row ? SHAP_BY_ROW : 0u)};
+      used += items * (c->shap_dm[leaf] >> 16);
+      runs.back().items = std::max(runs.back().items, items);
+    }
+    runs.back().t1 = t + 1;
+    largest = std::max(largest, used);
+  }
+  const size_t need = (size_t)largest * 8;
+  if (c->pm_shap_cap < need) {
+    c->pm_shap_cap = 0;  // dalloc frees the old workspace first
+    if ((rc = dalloc(c, &c->pm_shap, need))) return rc;
+    c->pm_shap_cap = need;
+  }
+  HIPCHK(c, hipMemcpyAsync(c->pm_splan, plan.data(), nleaf * sizeof(ShapPlan),
+                           hipMemcpyHostToDevice, c->stream));
+  const int64_t width = (int64_t)ntpi * (nf + 1);
+  for (int64_t r0 = 0; r0 < rows; r0 += chunk)
+    for (size_t i = 0; i < runs.size(); ++i) {
+      const Run& R = runs[i];
+      const PredTree& last = m->tree_index[(size_t)R.t1 - 1];
+      launch_shap_paths(c->pm_nodes, c->pm_trees, c->pm_leaves, c->pm_catb, c->pm_catw,
+                        c->pm_ncov, c->pm_lcov, c->pm_expv, c->pm_sleaf, c->pm_sstep,
+                        c->pm_sfeat, c->pm_splan, R.items, d_x + r0 * cols,
+                        std::min(chunk, rows - r0), cols, nf, max_leaves, R.t0, R.t1,
+                        m->tree_index[(size_t)R.t0].leaf0, last.leaf0 + last.num_leaves, ntpi,
+                        i == 0, (double*)c->pm_shap, d_out + r0 * width, c->stream);
+    }
+  HIPCHK(c, hipGetLastError());
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  return LGBM_HIP_OK;
+}
+
 int predict_run(lgbm_hip_ctx* c, const lgbm_hip_model* m, const float* d_x, int64_t rows,
                 int32_t cols, int32_t it0, int32_t it1, int32_t kind, void* d_out,
                 int32_t es_freq = 0, double es_margin = 0.0, int32_t* d_iters = nullptr) {
   if (kind == LGBM_HIP_PREDICT_CONTRIB) {
+    int32_t depth = 0, leaves = 1;
+    for (int64_t t = (int64_t)it0 * m->num_tree_per_iteration;
+         t < (int64_t)it1 * m->num_tree_per_iteration; ++t) {
+      depth = std::max(depth, m->tree_depth[t]);
+      leaves = std::max(leaves, m->tree_index[t].num_leaves);
+    }
+    if (it0 < it1 && depth <= SHAP_MAX_DEPTH && leaves <= SHAP_MAX_LEAVES &&
+        shap_rows_per_block(m->max_feature_idx + 1, leaves) > 0 &&
+        m->leaf_values.size() < (size_t)1 << 22)  // feature offsets fit 27 bits
+      return contrib_paths(c, m, d_x, rows, cols, it0, it1, leaves, (double*)d_out);
     // the deepest tree of the range sizes each row's path buffer; rows go in chunks
     // whose workspace stays within 256 MiB
-    int32_t depth = 0;
-    for (int64_t t = (int64_t)it0 * m->num_tree_per_iteration;
-         t < (int64_t)it1 * m->num_tree_per_iteration; ++t)
-      depth = std::max(depth, m->tree_depth[t]);
     const int64_t per_row = shap_bytes_per_row(depth);
     int64_t chunk = std::max<int64_t>(256, ((int64_t)256 << 20) / per_row / 256 * 256);
     chunk = std::min(chunk, rows);

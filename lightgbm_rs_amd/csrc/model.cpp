@@ -617,3 +617,59 @@ bool parse_model_text(const char* text, size_t len, lgbm_hip_model* m, std::stri
   m->uid = g_model_uid.fetch_add(1);
   return true;
 }
+
+void model_shap_paths(const lgbm_hip_model& m, ShapPaths* out) {
+  out->leaves.assign(m.leaf_values.size(), ShapLeaf{});
+  out->steps.clear();
+  out->feats.clear();
+  for (size_t t = 0; t < m.tree_index.size(); ++t) {
+    const PredTree& T = m.tree_index[t];
+    if (T.num_leaves <= 1 || T.num_leaves > SHAP_MAX_LEAVES || m.tree_depth[t] > SHAP_MAX_DEPTH)
+      continue;
+    const PredNode* nodes = m.nodes.data() + T.node0;
+    // leaves under each node: children after their parents in `order`, summed backwards
+    std::vector<int32_t> under((size_t)T.num_leaves - 1, 0), order{0};
+    for (size_t i = 0; i < order.size(); ++i)
+      for (const int32_t ch : {nodes[order[i]].left, nodes[order[i]].right})
+        if (ch >= 0) order.push_back(ch);
+    auto count = [&](int32_t ch) { return ch >= 0 ? under[(size_t)ch] : 1; };
+    for (size_t i = order.size(); i-- > 0;)
+      under[(size_t)order[i]] = count(nodes[order[i]].left) + count(nodes[order[i]].right);
+    // depth-first with the path so far: pending (node or leaf, its depth, the step to it)
+    struct Todo {
+      int32_t node, depth;
+      ShapStep step;
+    };
+    std::vector<ShapStep> path;
+    std::vector<Todo> todo{{0, 0, {}}};
+    while (!todo.empty()) {
+      const Todo d = todo.back();
+      todo.pop_back();
+      if (d.depth > 0) {
+        path.resize((size_t)d.depth - 1);
+        path.push_back(d.step);
+      }
+      if (d.node >= 0) {
+        const PredNode& n = nodes[d.node];
+        const int32_t at = T.node0 + d.node;
+        todo.push_back({n.right, d.depth + 1, {at, count(n.left) << 1 | 1}});
+        todo.push_back({n.left, d.depth + 1, {at, count(n.right) << 1}});
+        continue;
+      }
+      ShapLeaf& L = out->leaves[(size_t)T.leaf0 + (size_t)~d.node];
+      L.path0 = (int32_t)out->steps.size();
+      L.feat0 = (int32_t)out->feats.size();
+      L.tree = (int32_t)t;
+      // the unique path: a feature met again moves to its end
+      std::vector<int32_t> unique;
+      for (const ShapStep& s : path) {
+        const int32_t f = m.nodes[(size_t)s.node].feature;
+        unique.erase(std::remove(unique.begin(), unique.end(), f), unique.end());
+        unique.push_back(f);
+      }
+      L.dm = d.depth | (int32_t)unique.size() << 16;
+      out->steps.insert(out->steps.end(), path.begin(), path.end());
+      out->feats.insert(out->feats.end(), unique.begin(), unique.end());
+    }
+  }
+}

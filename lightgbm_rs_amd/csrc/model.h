@@ -39,6 +39,28 @@ struct PredLinLeaf {
   int32_t start, count;
 };
 
+// Feature contributions by leaf paths (k_shap_items, k_shap_rows).
+struct ShapLeaf {
+  int32_t path0;  // first of the leaf's ancestors (ShapStep), root first
+  int32_t feat0;  // first of the unique path's features
+  int32_t tree;
+  int32_t dm;     // depth | m << 16, m the unique path's length
+};
+struct ShapStep {
+  int32_t node;   // index into lgbm_hip_model::nodes
+  int32_t other;  // leaves of the child the path does not take, << 1 | 1 if it goes right
+};
+// Where a call's values of a leaf are: item i's m values at off + i * m; an item is a row
+// where `items` has SHAP_BY_ROW set, else an outcome of the leaf's ancestors.
+struct ShapPlan {
+  uint32_t off, items;
+};
+#define SHAP_BY_ROW 0x80000000u
+// The deepest and widest trees taken this way (one wave's LDS holds a path's weights, a
+// block's the leaves of its rows).
+constexpr int32_t SHAP_MAX_DEPTH = 31;
+constexpr int32_t SHAP_MAX_LEAVES = 1024;
+
 struct HostTree {
   int32_t num_leaves = 0, num_cat = 0;
   std::vector<int32_t> split_feature, left_child, right_child, decision_type, cat_boundaries;
@@ -91,3 +113,11 @@ std::string model_to_text(const lgbm_hip_model& m);
 bool model_add_tree(lgbm_hip_model* m, HostTree&& t, std::string* err);
 // Parses the objective line into m->objective / m->sigmoid.
 bool model_set_objective(lgbm_hip_model* m, const std::string& line, std::string* err);
+// Every leaf's path, by the index of its value; leaves of a tree that is deeper or wider
+// than the limits get none.
+struct ShapPaths {
+  std::vector<ShapLeaf> leaves;
+  std::vector<ShapStep> steps;
+  std::vector<int32_t> feats;
+};
+void model_shap_paths(const lgbm_hip_model& m, ShapPaths* out);
