@@ -144,6 +144,9 @@ struct lgbm_hip_ctx {
   PredLinLeaf* pm_linl = nullptr;
   int32_t* pm_linf = nullptr;
   double* pm_linc = nullptr;
+  PredEntry* pm_pack = nullptr;  // the packed trees of k_predict_lds (pack.words; NULL: none)
+  PredPack pack{};
+  bool pack_lds = false;  // the kernels were opted into their LDS
   double* pm_ncov = nullptr;  // TreeSHAP covers and expected values
   double* pm_lcov = nullptr;
   double* pm_expv = nullptr;
@@ -1482,6 +1485,7 @@ int lgbm_hip_ctx_destroy(lgbm_hip_ctx* c) {
   F(c->pm_lcov);
   F(c->pm_expv);
   F(c->pm_shap);
+  F(c->pm_pack);
   F(c->pm_sleaf);
   F(c->pm_sstep);
   F(c->pm_sfeat);
@@ -3342,6 +3346,15 @@ int predict_prepare(lgbm_hip_ctx* c, const lgbm_hip_model* m, int64_t rows, int3
     if ((rc = upload_vec(c, &c->pm_ncov, m->node_cover))) return rc;
     if ((rc = upload_vec(c, &c->pm_lcov, m->leaf_cover))) return rc;
     if ((rc = upload_vec(c, &c->pm_expv, m->tree_expected))) return rc;
+    PredPacked pk;
+    c->pack = PredPack{};
+    if (model_pack_trees(*m, &pk)) {
+      if (!c->pack_lds && predict_lds_prepare())
+        return set_err(c, LGBM_HIP_ERR_HIP, "the prediction kernels' LDS size was refused");
+      c->pack_lds = true;
+      if ((rc = upload_vec(c, &c->pm_pack, pk.words))) return rc;
+      c->pack = PredPack{(const uint2*)c->pm_pack, pk.stride, pk.values, pk.zero, pk.cat, pk.set};
+    }
     c->pm_uid = m->uid;
   }
   return LGBM_HIP_OK;
@@ -3434,6 +3447,22 @@ int contrib_paths(lgbm_hip_ctx* c, const lgbm_hip_model* m, const float* d_x, in
   return LGBM_HIP_OK;
 }
 
+// Enqueues k_predict_lds over R's rows.
+void predict_lds_run(lgbm_hip_ctx* c, const lgbm_hip_model* m, const PredShape& shape,
+                     const PredRows& R, bool csr, int64_t rows, int32_t width, int32_t it0,
+                     int32_t it1, int32_t kind, void* d_out) {
+  KernelEvents ke;
+  const bool leaf = kind == LGBM_HIP_PREDICT_LEAF;
+  launch_predict_lds(shape, c->pack, c->pm_catb, c->pm_catw, R, csr, rows, width, it0, it1,
+                     m->num_tree_per_iteration, kind, m->objective, m->sigmoid,
+                     m->average_output ? 1 : 0, leaf ? nullptr : (double*)d_out,
+                     leaf ? (int32_t*)d_out : nullptr, c->stream, ev_kernel(c, FAM_PRED, &ke));
+  if (c->timing) {
+    c->pred_launches += 1.0;
+    c->pred_walks += (double)rows * (double)(it1 - it0) * m->num_tree_per_iteration;
+  }
+}
+
 int predict_run(lgbm_hip_ctx* c, const lgbm_hip_model* m, const float* d_x, int64_t rows,
                 int32_t cols, int32_t it0, int32_t it1, int32_t kind, void* d_out,
                 int32_t es_freq = 0, double es_margin = 0.0, int32_t* d_iters = nullptr) {
@@ -3470,6 +3499,18 @@ int predict_run(lgbm_hip_ctx* c, const lgbm_hip_model* m, const float* d_x, int6
     return LGBM_HIP_OK;
   }
   KernelEvents ke;
+  const PredShape shape =
+      es_freq > 0 || !c->pack.words
+          ? PredShape{0, 0, 0}
+          : predict_lds_shape(rows, cols, c->pack.stride, (it1 - it0) * m->num_tree_per_iteration);
+  if (shape.rb > 0) {
+    PredRows R{};
+    R.dense = d_x;
+    predict_lds_run(c, m, shape, R, false, rows, cols, it0, it1, kind, d_out);
+    HIPCHK(c, hipGetLastError());
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return LGBM_HIP_OK;
+  }
   launch_predict(c->pm_nodes, c->pm_trees, c->pm_leaves, c->pm_catb, c->pm_catw, c->pm_linl,
                  c->pm_linf, c->pm_linc, d_x, rows, cols,
                  it0, it1, m->num_tree_per_iteration, kind, m->objective, m->sigmoid,
@@ -3563,7 +3604,13 @@ int predict_sparse(lgbm_hip_ctx* c, const lgbm_hip_model* m, const int64_t* indp
   int64_t* d_ptr = (int64_t*)(c->pm_csr + 256);
   int32_t* d_idx = (int32_t*)(c->pm_csr + 256 + pb);
   float* d_val = (float*)(c->pm_csr + 256 + pb + ib);
-  const size_t xb = (size_t)num_rows * (size_t)std::max(fw, 1) * 4;
+  // CSR rows go straight into k_predict_lds's LDS where they fit
+  const PredShape shape =
+      csc || kind == LGBM_HIP_PREDICT_CONTRIB || !c->pack.words
+          ? PredShape{0, 0, 0}
+          : predict_lds_shape(num_rows, fw, c->pack.stride, (it1 - it0) * m->num_tree_per_iteration);
+  const bool direct = shape.rb > 0;
+  const size_t xb = direct ? 0 : (size_t)num_rows * (size_t)std::max(fw, 1) * 4;
   const size_t ob = (size_t)num_rows * (size_t)width * (kind == LGBM_HIP_PREDICT_LEAF ? 4 : 8);
   if (c->pm_x_cap < xb) {
     c->pm_x_cap = 0;  // dalloc frees the old staging first
@@ -3584,8 +3631,18 @@ int predict_sparse(lgbm_hip_ctx* c, const lgbm_hip_model* m, const int64_t* indp
     HIPCHK(c, hipMemcpy(d_idx, indices, ib, hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(d_val, values, ib, hipMemcpyHostToDevice));
   }
-  HIPCHK(c, hipMemsetAsync(c->pm_x, 0, (size_t)num_rows * (size_t)fw * 4, c->stream));
-  if (csc) {
+  if (!direct)
+    HIPCHK(c, hipMemsetAsync(c->pm_x, 0, (size_t)num_rows * (size_t)fw * 4, c->stream));
+  if (direct) {
+    PredRows R{};
+    R.indptr = d_ptr;
+    R.indices = d_idx;
+    R.values = d_val;
+    R.nnz = nnz;
+    R.cols = num_cols;
+    R.err = d_err;
+    predict_lds_run(c, m, shape, R, true, num_rows, fw, it0, it1, kind, c->pm_out);
+  } else if (csc) {
     launch_csc_dense(d_ptr, d_idx, d_val, nnz, num_rows, num_cols, fw, c->pm_x, d_err, c->stream);
   } else {
     launch_csr_dense(d_ptr, d_idx, d_val, nnz, num_rows, num_cols, fw, c->pm_x, d_err, c->stream);
@@ -3598,7 +3655,9 @@ int predict_sparse(lgbm_hip_ctx* c, const lgbm_hip_model* m, const int64_t* indp
   if (bad & 2u)
     return set_err(c, LGBM_HIP_ERR_LENGTH_MISMATCH,
                    csc ? "csc row index out of range" : "csr column index out of range");
-  if ((rc = predict_run(c, m, c->pm_x, num_rows, fw, it0, it1, kind, c->pm_out))) return rc;
+  if (!direct &&
+      (rc = predict_run(c, m, c->pm_x, num_rows, fw, it0, it1, kind, c->pm_out)))
+    return rc;
   HIPCHK(c, hipMemcpy(out, c->pm_out, ob, hipMemcpyDeviceToHost));
   return LGBM_HIP_OK;
 }

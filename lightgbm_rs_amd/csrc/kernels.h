@@ -223,6 +223,32 @@ struct DevBinFeature {
 void launch_bin_records(const void* x, int32_t f64, int32_t col_major, int64_t n, int32_t F,
                         int32_t fmt, const DevBinFeature* feats, const double* ub, int32_t ub_count,
                         const int2* cats, uint4* rec, hipStream_t s, const KernelEvents* ev);
+// k_predict_lds: the packed trees (model_pack_trees), where its rows come from, and a launch's shape.
+struct PredPack {
+  const uint2* words;
+  int32_t stride, values;
+  int32_t zero, cat, set;
+};
+struct PredRows {
+  const float* dense;     // rows of `width` floats, or
+  const int64_t* indptr;  // CSR over `cols` columns
+  const int32_t* indices;
+  const float* values;
+  int64_t nnz;
+  int32_t cols;
+  uint32_t* err;  // bit 0: a bad indptr pair, bit 1: a bad column
+};
+struct PredShape {
+  int32_t rb, nb;  // rows and staged trees of a block
+  size_t lds;
+};
+PredShape predict_lds_shape(int64_t rows, int32_t width, int32_t tree_words, int32_t n_trees);
+int predict_lds_prepare();
+void launch_predict_lds(const PredShape& S, const PredPack& K, const int32_t* cat_bounds,
+                        const uint32_t* cat_words, const PredRows& R, bool csr, int64_t rows,
+                        int32_t width, int32_t it0, int32_t it1, int32_t ntpi, int32_t kind,
+                        int32_t objective, double sigmoid, int32_t average_output, double* out,
+                        int32_t* leaf_out, hipStream_t s, const KernelEvents* ev);
 void launch_absmax(const float* g, const float* h, int64_t n, uint4* partials, hipStream_t s);
 void launch_grad_binary(const double* score, const float* label, float* g, float* h, int64_t n,
                         uint4* partials, hipStream_t s);

@@ -39,6 +39,26 @@ struct PredLinLeaf {
   int32_t start, count;
 };
 
+// A tree as k_predict_lds walks it: `stride` 8-byte words, its entries (nodes and leaves,
+// children neighbours, the root first) and from word `values` on its leaf values (f64).
+// A node's word holds its first child (low 16 bits) and feature (12 bits); the walk goes
+// on to the second child where (v with its sign flipped if PRED_FLIP is set) > threshold.
+// Children are stored right first with PRED_FLIP and left first without, so that a NaN,
+// for which the comparison fails, goes the node's way for it; with PRED_ZERO_MISSING a
+// value within 1e-35 of zero is taken for a NaN.  A PRED_CATEGORICAL node's first child
+// is the left one and its threshold the set of categories 0 to 31 that go there, or with
+// PRED_SET the set's index in cat_bounds.  A leaf has first child 0 and its number in the
+// threshold.
+#define PRED_CATEGORICAL (1u << 28)
+#define PRED_SET (1u << 29)
+#define PRED_ZERO_MISSING (1u << 30)
+#define PRED_FLIP (1u << 31)
+constexpr int32_t PRED_TREE_WORDS = 4096;  // of a tree at most, and of a staged batch
+struct PredEntry {
+  float threshold;
+  uint32_t word;
+};
+
 // Feature contributions by leaf paths (k_shap_items, k_shap_rows).
 struct ShapLeaf {
   int32_t path0;  // first of the leaf's ancestors (ShapStep), root first
@@ -121,3 +141,12 @@ struct ShapPaths {
   std::vector<int32_t> feats;
 };
 void model_shap_paths(const lgbm_hip_model& m, ShapPaths* out);
+// Every tree's entries and leaf values, `stride` words a tree; false where a tree or
+// feature is too large for the form, a leaf is linear or a threshold infinite or NaN.
+struct PredPacked {
+  std::vector<PredEntry> words;
+  int32_t stride = 0, values = 0;
+  // whether any node has PRED_ZERO_MISSING, PRED_CATEGORICAL, PRED_SET
+  bool zero = false, cat = false, set = false;
+};
+bool model_pack_trees(const lgbm_hip_model& m, PredPacked* out);
