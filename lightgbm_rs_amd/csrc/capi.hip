@@ -134,6 +134,7 @@ struct FeatureSampler {
 }  // namespace
 
 struct lgbm_hip_ctx {
+  size_t label_cap = 0, score_cap = 0, gk_cap = 0, hk_cap = 0;  // elements (dkeep)
   // device copy of the last model predicted with (keyed by the model's uid)
   uint64_t pm_uid = 0;
   PredNode* pm_nodes = nullptr;
@@ -360,6 +361,16 @@ int dalloc(lgbm_hip_ctx* c, T** p, size_t count) {
   if (count == 0) count = 1;
   HIPCHK(c, hipMalloc((void**)p, count * sizeof(T)));
   return LGBM_HIP_OK;
+}
+
+// dalloc for a buffer that training calls size anew: kept while its size stays the same.
+template <typename T>
+int dkeep(lgbm_hip_ctx* c, T** p, size_t* cap, size_t count) {
+  if (*p && *cap == count) return LGBM_HIP_OK;
+  *cap = 0;
+  const int rc = dalloc(c, p, count);
+  if (!rc) *cap = count;
+  return rc;
 }
 
 // ---- xorshift64 jump matrices (GF(2)); column i = image of basis vector e_i ----
@@ -2599,11 +2610,15 @@ int lgbm_hip_set_labels(lgbm_hip_ctx* c, const float* labels, int64_t n, double 
   if (!c->have_bins) return set_err(c, LGBM_HIP_ERR_RUNTIME, "upload bins first");
   if (!labels) return set_err(c, LGBM_HIP_ERR_INVALID_ARGUMENT, "null labels");
   if (n != c->N) return set_err(c, LGBM_HIP_ERR_LENGTH_MISMATCH, "labels length != num_data");
-  if ((rc = dalloc(c, &c->label, (size_t)n))) return rc;
-  if ((rc = dalloc(c, &c->score, (size_t)n))) return rc;
+  // a lookahead left queued by train_iter reads the old labels and scores
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  c->have_labels = false;
+  if ((rc = dkeep(c, &c->label, &c->label_cap, (size_t)n))) return rc;
+  if ((rc = dkeep(c, &c->score, &c->score_cap, (size_t)n))) return rc;
   HIPCHK(c, hipMemcpy(c->label, labels, (size_t)n * 4, hipMemcpyHostToDevice));
-  std::vector<double> s((size_t)n, init_score);
-  HIPCHK(c, hipMemcpy(c->score, s.data(), (size_t)n * 8, hipMemcpyHostToDevice));
+  launch_fill(c->score, n, init_score, c->stream);
+  HIPCHK(c, hipGetLastError());
+  HIPCHK(c, hipStreamSynchronize(c->stream));
   c->num_class = 1;
   c->have_labels = true;
   c->have_rank = false;  // the lambdarank tables were built from the old labels
@@ -2898,18 +2913,18 @@ int lgbm_hip_set_labels_multiclass(lgbm_hip_ctx* c, const float* labels, int64_t
                      "label " + std::to_string(l) + " at row " + std::to_string(i) +
                          " is not a class in [0, num_class)");
   }
+  HIPCHK(c, hipStreamSynchronize(c->stream));
   c->have_labels = false;
   const size_t kn = (size_t)num_class * (size_t)n;
-  if ((rc = dalloc(c, &c->label, (size_t)n))) return rc;
-  if ((rc = dalloc(c, &c->score, kn))) return rc;
-  if ((rc = dalloc(c, &c->gk, kn))) return rc;
-  if ((rc = dalloc(c, &c->hk, kn))) return rc;
+  if ((rc = dkeep(c, &c->label, &c->label_cap, (size_t)n))) return rc;
+  if ((rc = dkeep(c, &c->score, &c->score_cap, kn))) return rc;
+  if ((rc = dkeep(c, &c->gk, &c->gk_cap, kn))) return rc;
+  if ((rc = dkeep(c, &c->hk, &c->hk_cap, kn))) return rc;
   HIPCHK(c, hipMemcpy(c->label, labels, (size_t)n * 4, hipMemcpyHostToDevice));
-  std::vector<double> s(kn, 0.0);
-  if (init_scores)
-    for (int32_t k = 0; k < num_class; ++k)
-      std::fill(s.begin() + (size_t)k * n, s.begin() + (size_t)(k + 1) * n, init_scores[k]);
-  HIPCHK(c, hipMemcpy(c->score, s.data(), kn * 8, hipMemcpyHostToDevice));
+  for (int32_t k = 0; k < num_class; ++k)
+    launch_fill(c->score + (size_t)k * n, n, init_scores ? init_scores[k] : 0.0, c->stream);
+  HIPCHK(c, hipGetLastError());
+  HIPCHK(c, hipStreamSynchronize(c->stream));
   c->num_class = num_class;
   c->have_labels = true;
   c->have_rank = false;

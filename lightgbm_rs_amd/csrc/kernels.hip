@@ -1025,6 +1025,13 @@ __global__ void k_pack_partition(const uint32_t* __restrict__ bins, int64_t n,
   if (i < n) rec[i] = make_uint4(bins[i] & 0xffu, 0u, 0u, (uint32_t)i);
 }
 
+// The training score's reset.  From a host vector it cost that vector's fill and a copy:
+// 37.6 ms a call for 2M rows x 10 classes, against 40 us of stores here.
+__global__ __launch_bounds__(256) void k_fill(double* __restrict__ dst, int64_t n, double v) {
+  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) dst[i] = v;
+}
+
 // Timing pass only: one wave that waits `ticks` of the constant-rate wall clock (a
 // second bound, 2^20 sleeps of ~3 us, ends it whatever the clock reads), so that the
 // host has enqueued the whole kernel sequence behind it before the device starts it.
@@ -1223,6 +1230,12 @@ void launch_pack_partition(const uint32_t* bins, int64_t n, uint4* rec, hipStrea
   const int64_t blocks = (n + 255) / 256;
   if (blocks < 1) return;
   k_pack_partition<<<dim3((unsigned)blocks), dim3(256), 0, s>>>(bins, n, rec);
+}
+
+void launch_fill(double* dst, int64_t n, double v, hipStream_t s) {
+  const int64_t blocks = std::min<int64_t>((n + 255) / 256, 4096);
+  if (blocks < 1) return;
+  k_fill<<<dim3((unsigned)blocks), dim3(256), 0, s>>>(dst, n, v);
 }
 
 void launch_hold(uint64_t ticks, hipStream_t s) {
