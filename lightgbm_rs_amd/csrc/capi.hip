@@ -226,7 +226,8 @@ struct lgbm_hip_ctx {
   int32_t* hist_sum = nullptr;   // [cells][3]
   int32_t* hist_acc = nullptr;   // [SPEC_MAX][acc_cells][3]
   unsigned long long* hist_accp = nullptr;  // [SPEC_MAX][acc_cells] packed (small jobs)
-  int64_t* hist_acc64 = nullptr;  // wide layout: [SPEC_MAX][acc_cells][2]
+  int64_t* hist_acc64 = nullptr;  // [SPEC_MAX][acc_cells][2]
+  int64_t* hist_sum64 = nullptr;  // [cells][2]
   unsigned long long* wide_part = nullptr;  // wide layout: per-chunk partial cells
   int32_t acc_cells = 0;          // total_cells (+ 1 totals cell in the wide layout)
   unsigned long long* part_slots = nullptr;  // [part_blocks + SPEC_MAX][cells] packed
@@ -438,6 +439,7 @@ DevLearner make_learner(lgbm_hip_ctx* c) {
   L.hist_sum = c->hist_sum;
   L.hist_acc = c->hist_acc;
   L.hist_acc64 = c->hist_acc64;
+  L.hist_sum64 = c->hist_sum64;
   L.hist_accp = c->hist_accp;
   L.wide_part = c->wide_part;
   L.acc_cells = c->acc_cells;
@@ -739,7 +741,7 @@ void enqueue_rounds(lgbm_hip_ctx* c, int32_t rounds, int32_t fp) {
     launch_partition(L, fp, c->part_blocks, c->stream, ev_kernel(c, FAM_PART, &ke));
     if (rec_wide(c->fmt))
       launch_hist_wide(L, fp, c->stream, ev_kernel(c, FAM_HIST, &ke));
-    else if (fp)
+    else if (fp && c->N > HIST_FP_ALL_DIRECT)
       launch_hist_f32(L, c->stream, ev_kernel(c, FAM_HIST, &ke));
     launch_pair_scan(L, fp, c->spec_max, c->part_blocks, c->stream, ev_kernel(c, FAM_SCAN, &ke));
   }
@@ -758,7 +760,7 @@ void enqueue_tree(lgbm_hip_ctx* c, int32_t num_leaves, int32_t max_depth, int32_
     launch_hist_f32(L, c->stream, ev_kernel(c, FAM_HIST, &ke));
   else
     launch_hist(L, c->stream, ev_kernel(c, FAM_HIST, &ke));
-  launch_fixscan(L, 1, nullptr, c->stream, ev_kernel(c, FAM_SCAN, &ke));
+  launch_fixscan(L, fp, 1, nullptr, c->stream, ev_kernel(c, FAM_SCAN, &ke));
   enqueue_rounds(c, rounds, fp);
 }
 
@@ -1247,8 +1249,6 @@ int resident_setup(lgbm_hip_ctx* c, int32_t F_in, int64_t num_data, const lgbm_f
     c->n_wgroups = (int32_t)groups.size() - 1;
     if ((rc = dalloc(c, &c->d_wgroups, groups.size()))) return rc;
     HIPCHK(c, hipMemcpy(c->d_wgroups, groups.data(), groups.size() * 4, hipMemcpyHostToDevice));
-    if ((rc = dalloc(c, &c->hist_acc64, (size_t)SPEC_MAX * c->acc_cells * 2))) return rc;
-    HIPCHK(c, hipMemset(c->hist_acc64, 0, (size_t)SPEC_MAX * c->acc_cells * 2 * 8));
     if ((rc = dalloc(c, &c->wide_part,
                      wide_part_words(F, num_data, (int32_t)acc, bin16 ? c->n_wgroups : 0))))
       return rc;
@@ -1256,11 +1256,9 @@ int resident_setup(lgbm_hip_ctx* c, int32_t F_in, int64_t num_data, const lgbm_f
     c->row_stride = 0;
     if (c->binmat) (void)hipFree(c->binmat);
     if (c->bincol) (void)hipFree(c->bincol);
-    if (c->hist_acc64) (void)hipFree(c->hist_acc64);
     if (c->wide_part) (void)hipFree(c->wide_part);
     c->binmat = nullptr;
     c->bincol = nullptr;
-    c->hist_acc64 = nullptr;
     c->wide_part = nullptr;
     if (acc > (uint32_t)(MAX_FGROUPS - 1) * (HIST_FP_CELLS - 256))
       return set_err(c, LGBM_HIP_ERR_CAPABILITY, "too many histogram cells for the f32 feature groups");
@@ -1284,6 +1282,9 @@ int resident_setup(lgbm_hip_ctx* c, int32_t F_in, int64_t num_data, const lgbm_f
     c->fgroup_first[++ng] = F;
     c->n_fgroups = ng;
   }
+  if ((rc = dalloc(c, &c->hist_sum64, (size_t)acc * 2))) return rc;
+  if ((rc = dalloc(c, &c->hist_acc64, (size_t)SPEC_MAX * c->acc_cells * 2))) return rc;
+  HIPCHK(c, hipMemset(c->hist_acc64, 0, (size_t)SPEC_MAX * c->acc_cells * 2 * 8));
   if ((rc = dalloc(c, &c->hist_acc, (size_t)SPEC_MAX * c->acc_cells * 3))) return rc;
   HIPCHK(c, hipMemset(c->hist_acc, 0, (size_t)SPEC_MAX * c->acc_cells * 3 * 4));
   if ((rc = dalloc(c, &c->hist_accp, (size_t)SPEC_MAX * c->acc_cells))) return rc;
@@ -1437,6 +1438,7 @@ int lgbm_hip_ctx_destroy(lgbm_hip_ctx* c) {
   F(c->hist_acc);
   F(c->hist_accp);
   F(c->hist_acc64);
+  F(c->hist_sum64);
   F(c->wide_part);
   F(c->d_wgroups);
   F(c->binmat);
@@ -2061,7 +2063,7 @@ static int set_hist_job(lgbm_hip_ctx* c, const uint32_t* rows, int64_t n_rows) {
     buf = BUF_S0;
     count = n_rows;
   }
-  const HistJob hj{buf, 0, 0, count, 0, 0};
+  const HistJob hj{buf, 1, 0, count, 0, 0};  // _pad bit 0: partial slots, as the root's
   if ((rc = ctl_write(c, CTL_OFF(hjobs), hj))) return rc;
   const int32_t one = 1;
   if ((rc = ctl_write(c, CTL_OFF(n_hjobs), one))) return rc;
@@ -2148,7 +2150,7 @@ static int build_leaf_into(lgbm_hip_ctx* c, const uint32_t* leaf_rows, int64_t n
     launch_hist_f32(L, c->stream);
   else
     launch_hist(L, c->stream);
-  launch_fixscan(L, 2, d_out, c->stream);
+  launch_fixscan(L, fp, 2, d_out, c->stream);
   HIPCHK(c, hipGetLastError());
   return LGBM_HIP_OK;
 }

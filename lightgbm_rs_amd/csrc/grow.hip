@@ -84,6 +84,8 @@ __global__ void k_tree_init(DevLearner L, int32_t max_leaves, int32_t max_depth,
         L.hist_acc[3 * t + 2] = 0;
       }
     }
+  } else if (fp_mode) {
+    for (int i = tid; i < SPEC_MAX * L.acc_cells * 2; i += nthr) L.hist_acc64[i] = 0;
   } else {
     for (int i = tid; i < SPEC_MAX * L.acc_cells * 3; i += nthr) L.hist_acc[i] = 0;
     for (int i = tid; i < SPEC_MAX * L.acc_cells; i += nthr) L.hist_accp[i] = 0ull;
@@ -1093,11 +1095,13 @@ __global__ __launch_bounds__(PART_THREADS) void k_partition(DevLearner L) {
           hj.buf = J.dst_buf;
           hj._pad = 0;
           hj.begin = right ? begin + lc : begin;
-          hj.count = gated ? 0 : (right ? rc : lc);
+          const int32_t built = gated ? 0 : (right ? rc : lc);
+          // the record layouts' small f32 children are built by the scan itself
+          hj.count = FP && !WIDE && built <= hist_fp_direct(L.N) ? 0 : built;
           hj.a0 = 0;
           hj.nblk = 0;
           ctl->hjobs[j] = hj;
-          atomicAdd(&L.stats[5], (double)hj.count);  // rows of the child builds
+          atomicAdd(&L.stats[5], (double)built);  // rows of the child builds
         }
         atomicAdd(&L.stats[0], (double)count);
         atomicAdd(&L.stats[4], 1.0);
@@ -1265,8 +1269,12 @@ __global__ __launch_bounds__(SCAN_THREADS, 6) void k_pair_scan(DevLearner L, int
   if (pgate && !gated && (fp_mode || wide)) {
     // The parent cannot split on this feature (outside the column sample, or no
     // valid threshold), so neither child scans it and no descendant reads its cells;
-    // these layouts hold no accumulator to clear (their partial slots are rewritten
-    // every round).  The children get what the scan below would give them.
+    // only an accumulator of the record layouts' f32 builds is cleared (partial slots are
+    // rewritten every round).  The children get what the scan below would give them.
+    if (fp_mode && !wide && ctl->hjobs[j].nblk > HIST_FP_SLOTS) {
+      longlong2* acc = (longlong2*)L.hist_acc64 + (size_t)j * L.acc_cells + ft.cell_base;
+      for (int b = tid; b < nb; b += SCAN_THREADS) acc[b] = make_longlong2(0, 0);
+    }
     if (tid == 0 || tid == LGBM_WAVE) {
       const int32_t leaf = tid == 0 ? sm : lg;
       const LeafSums ls = (tid == 0) == right_small ? scr : scl;
@@ -1282,11 +1290,55 @@ __global__ __launch_bounds__(SCAN_THREADS, 6) void k_pair_scan(DevLearner L, int
     // fixed point
     const int32_t a0 = ctl->hjobs[j].a0, na = ctl->hjobs[j].nblk;
     const double gu = ldexp(1.0, -ctl->g_shift), hu = ldexp(1.0, -ctl->h_shift);
+    const int32_t scnt = right_small ? rcnt : lcnt;
+    const bool direct = !wide && scnt <= hist_fp_direct(L.N);
+    if (!gated && direct) {
+      // a small child: its rows' bins of this feature, added here (k_hist_f32 would take
+      // a whole pass over its LDS cells for a few hundred rows); the fixed-point cells
+      // stand in cs until the loop below turns them into f64
+      unsigned long long* cell = (unsigned long long*)cs;
+      for (int i = tid; i < 2 * nb; i += SCAN_THREADS) cell[i] = 0ull;
+      __syncthreads();
+      const int fmt = L.fmt, U = rec_words(fmt);
+      int wi, sh;
+      rec_field_pos(fmt, f, &wi, &sh);
+      const uint32_t mask = (1u << rec_bits(fmt)) - 1u;
+      const int32_t buf = nd.buf[sm];
+      const int64_t begin = nd.begin[sm];
+      const uint32_t* __restrict__ rec = (const uint32_t*)rec_buf(L.bufs, buf) + begin * U + wi;
+      const float2* __restrict__ gh = buf_sel(L.bufs.g32, buf) + begin;
+      const double gm = ldexp(1.0, ctl->g_shift), hm = ldexp(1.0, ctl->h_shift);
+      constexpr int RU = 4;
+      for (int32_t r0 = tid; r0 < scnt; r0 += RU * SCAN_THREADS) {
+        uint32_t w[RU];
+        float2 v[RU];
+#pragma unroll
+        for (int u = 0; u < RU; ++u) {
+          const int32_t r = min(r0 + u * SCAN_THREADS, scnt - 1);
+          w[u] = rec[(int64_t)r * U];
+          v[u] = gh[r];
+        }
+#pragma unroll
+        for (int u = 0; u < RU; ++u) {
+          if (r0 + u * SCAN_THREADS >= scnt) continue;
+          const uint32_t b = (w[u] >> sh) & mask;
+          __hip_atomic_fetch_add(&cell[2 * b], (unsigned long long)(long long)rint((double)v[u].x * gm),
+                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          __hip_atomic_fetch_add(&cell[2 * b + 1],
+                                 (unsigned long long)(long long)rint((double)v[u].y * hm),
+                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+      }
+      __syncthreads();
+    }
     if (!gated) {
       for (int b = tid; b < nb; b += SCAN_THREADS) {
         const size_t ci = (size_t)(ft.cell_base + b);
         long long SG = 0, SH = 0;
-        if (wide) {
+        if (direct) {
+          SG = ((const long long*)cs)[2 * b];
+          SH = ((const long long*)cs)[2 * b + 1];
+        } else if (wide) {
           // the job's chunks, four loads in flight at a time (integer sums: any order)
           const ulonglong2* wp = (const ulonglong2*)L.wide_part + (size_t)a0 * cells + ci;
           int k = 0;
@@ -1306,7 +1358,7 @@ __global__ __launch_bounds__(SCAN_THREADS, 6) void k_pair_scan(DevLearner L, int
             SH += (long long)x.y;
           }
         } else {
-          hist_part_sum64(L, a0, na, ci, &SG, &SH);
+          hist_child_sum64(L, j, a0, na, ci, &SG, &SH);
         }
         const int64_t* ps = L.int_slots64 + ((size_t)p * cells + ci) * 2;
         int64_t* sp_ = L.int_slots64 + ((size_t)sm * cells + ci) * 2;

@@ -120,7 +120,9 @@ struct DevLearner {
   int32_t* hist_sum;          // [total_cells][3] job 0's partials summed (k_hist_reduce)
   int32_t* hist_acc;          // [SPEC_MAX][acc_cells][3] per-job accumulators
   unsigned long long* hist_accp;  // [SPEC_MAX][acc_cells] packed accumulators (small jobs)
-  int64_t* hist_acc64;        // wide layout, f32 gradients: [SPEC_MAX][acc_cells][2]
+  int64_t* hist_sum64;        // [total_cells][2] the same of the f32 slots (k_hist_reduce64)
+  int64_t* hist_acc64;        // f32 gradients: [SPEC_MAX][acc_cells][2] per-job accumulators
+                              // (the wide layout's hold the root's row totals only)
   unsigned long long* wide_part;  // wide layout: per-chunk partial cells [chunks][cells][1 or 2]
   int32_t acc_cells;          // cells per accumulator: total_cells, + 1 (row totals) when wide
   const uint8_t* binmat;      // wide layout: row-major bins [N][row_stride]
@@ -268,7 +270,7 @@ void launch_quantize(const float* g, const float* h, int64_t n, const Ctl* ctl,
 void launch_requant(const float* g, const float* h, int64_t n, const Ctl* ctl, int32_t bins,
                     uint16_t* gh, unsigned long long* bad, hipStream_t s);
 void launch_hist(const DevLearner& L, hipStream_t s, const KernelEvents* ev = nullptr);
-void launch_fixscan(const DevLearner& L, int32_t mode, double* explicit_out, hipStream_t s,
+void launch_fixscan(const DevLearner& L, int fp, int32_t mode, double* explicit_out, hipStream_t s,
                     const KernelEvents* ev = nullptr);
 void launch_plan(const DevLearner& L, int32_t slot_cap, hipStream_t s,
                  const KernelEvents* ev = nullptr);

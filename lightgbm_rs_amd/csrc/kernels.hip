@@ -658,16 +658,56 @@ __global__ __launch_bounds__(256) void k_hist_reduce(DevLearner L) {
   }
 }
 
+// The same of the 64-bit fixed-point slots (f32 gradients), into L.hist_sum64.
+__global__ __launch_bounds__(256) void k_hist_reduce64(DevLearner L) {
+  __shared__ long long part[16][17];
+  const Ctl* ctl = L.ctl;
+  const int32_t a0 = ctl->hjobs[0].a0, na = ctl->n_hjobs > 0 ? ctl->hjobs[0].nblk : 0;
+  const int64_t ncol = (int64_t)L.total_cells * 2;
+  const int cl = threadIdx.x & 15, g = threadIdx.x >> 4;
+  const int64_t col = (int64_t)blockIdx.x * 16 + cl;
+  long long s = 0;
+  if (col < ncol) {
+    const int64_t* p = L.hist_part64 + (size_t)a0 * ncol + col;
+    long long x[4] = {0, 0, 0, 0};
+    int k = g;
+    for (; k + 48 < na; k += 64) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) x[u] += p[(size_t)(k + 16 * u) * ncol];
+    }
+    for (; k < na; k += 16) x[0] += p[(size_t)k * ncol];
+    s = (x[0] + x[1]) + (x[2] + x[3]);
+  }
+  part[g][cl] = s;
+  __syncthreads();
+  if (g == 0 && col < ncol) {
+    long long t = 0;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) t += part[k][cl];
+    L.hist_sum64[col] = t;
+  }
+}
+
 // f32 gradients: ConstructHistogram of the histogram jobs into 64-bit fixed-point
 // (g, h) cells with 64-bit LDS atomics (exact, order-independent).  Block (chunk a,
-// feature group y): the rows of chunk a (hist_assign) and the features of group y,
-// whose cells fit LDS; partial slot a receives the group's cells.
+// feature group y): the rows of chunk a and the features of group y, whose cells fit
+// LDS (two blocks a CU).  The root's chunks, and those of a child job cut into at most
+// HIST_FP_SLOTS, store their cells in partial slot a; a wider child job's add them into
+// the job's accumulator (L.hist_acc64, read and cleared by k_pair_scan), whose reader
+// would else sum hundreds of slots one by one.
+//
+// The features of a group are walked with their word, shift and first cell known at
+// compile time or in scalar registers: two atomics and four VALU instructions a (row,
+// feature).  Read from LDS tables per feature, with the word picked by masking them all,
+// it was bound by VALU: 1M rows x 28 features of 255 bins, all builds of a tree of 63
+// leaves, 613 us.
 template <int FMT>
-__global__ __launch_bounds__(HIST_THREADS) void k_hist_f32(DevLearner L) {
-  constexpr int U = rec_words(FMT);
-  extern __shared__ unsigned long long lds64[];
-  __shared__ int32_t cb[16 * LGBM_MAX_W];
-  __shared__ int32_t s_pos[16 * LGBM_MAX_W];  // feature f's field: word << 8 | shift
+__global__ __launch_bounds__(HIST_THREADS, 2) void k_hist_f32(DevLearner L) {
+  constexpr int U = rec_words(FMT), BPW = rec_bpw(FMT), BB = rec_bits(FMT), NS = rec_slots(FMT);
+  constexpr uint32_t BM = (1u << BB) - 1u;
+  constexpr int RU = 2;  // rows a thread has in flight
+  extern __shared__ __align__(16) unsigned long long lds64[];
+  __shared__ int32_t cb[NS];
   __shared__ int32_t s_a0[SPEC_MAX], s_nb[SPEC_MAX];
   __shared__ int64_t s_R;
   Ctl* ctl = L.ctl;
@@ -677,20 +717,27 @@ __global__ __launch_bounds__(HIST_THREADS) void k_hist_f32(DevLearner L) {
   const int tid = threadIdx.x;
   const int cells = L.total_cells;
   const int f0 = L.fgroup_first[grp], f1 = L.fgroup_first[grp + 1];
-  if (tid == 0) {
-    hist_assign(ctl, nj, s_a0, s_nb, &s_R, HIST_GRID);
-    if (blockIdx.x == 0 && grp == 0)
-      for (int j = 0; j < nj; ++j) {
-        ctl->hjobs[j].a0 = s_a0[j];
-        ctl->hjobs[j].nblk = s_nb[j];
+  if (tid < LGBM_WAVE) {
+    // lane j = job j: chunks of R rows, the first chunk of every job
+    const int lane = tid;
+    const int64_t c = lane < nj ? max(ctl->hjobs[lane].count, (int64_t)0) : 0;
+    int64_t S = c;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) S += __shfl_xor(S, off);
+    const int64_t R = max((S + HIST_GRID - 1) / HIST_GRID, (int64_t)HIST_FP_MIN_ROWS);
+    const int32_t nb = c > 0 ? (int32_t)((c + R - 1) / R) : 0;
+    const int32_t incl = wave_incl_sum_i32(nb);
+    if (lane < nj) {
+      s_a0[lane] = incl - nb;
+      s_nb[lane] = nb;
+      if (blockIdx.x == 0 && grp == 0) {  // the readers' chunk ranges
+        ctl->hjobs[lane].a0 = incl - nb;
+        ctl->hjobs[lane].nblk = nb;
       }
+    }
+    if (lane == 0) s_R = R;
   }
-  for (int f = f0 + tid; f < f1; f += HIST_THREADS) {
-    cb[f] = (int32_t)L.feats[f].cell_base;
-    int wi, sh;
-    rec_field_pos(FMT, f, &wi, &sh);
-    s_pos[f] = (wi << 8) | sh;
-  }
+  for (int f = tid; f < NS; f += HIST_THREADS) cb[f] = f < L.F ? (int32_t)L.feats[f].cell_base : 0;
   __syncthreads();
   const int32_t a = (int32_t)blockIdx.x;
   int32_t j = -1;
@@ -698,33 +745,55 @@ __global__ __launch_bounds__(HIST_THREADS) void k_hist_f32(DevLearner L) {
     if (a >= s_a0[k] && a < s_a0[k] + s_nb[k]) j = k;
   if (j < 0) return;
   const int cbase = cb[f0];
-  const int gcells = (f1 < L.F ? (int)L.feats[f1].cell_base : cells) - cbase;
-  for (int c = tid; c < 2 * gcells; c += HIST_THREADS) lds64[c] = 0ull;
+  const int gcells = (f1 < L.F ? cb[f1] : cells) - cbase;
+  for (int c = tid; c < gcells; c += HIST_THREADS) ((ulonglong2*)lds64)[c] = make_ulonglong2(0ull, 0ull);
+  int32_t cbr[NS];  // the group's first cells, in LDS
+#pragma unroll
+  for (int f = 0; f < NS; ++f) cbr[f] = __builtin_amdgcn_readfirstlane(cb[f]) - cbase;
   __syncthreads();
   const HistJob& J = ctl->hjobs[j];
   const int64_t R = s_R;
   const int64_t lo = (int64_t)(a - s_a0[j]) * R;
   const int64_t hi = min(J.count, lo + R);
   const uint4* __restrict__ rec = rec_buf(L.bufs, J.buf);  // rows J.begin + r
-  const float2* __restrict__ gh = L.bufs.g32[J.buf] + J.begin;
+  const float2* __restrict__ gh = buf_sel(L.bufs.g32, J.buf) + J.begin;
   const int64_t rb = J.begin;
   const double gm = ldexp(1.0, ctl->g_shift), hm = ldexp(1.0, ctl->h_shift);
-  for (int64_t r = lo + tid; r < hi; r += HIST_THREADS) {
-    uint32_t w[U];
-    rec_load<FMT>(rec, rb + r, w);
-    const float2 v = gh[r];
-    const unsigned long long gi = (unsigned long long)(long long)rint((double)v.x * gm);
-    const unsigned long long hi_ = (unsigned long long)(long long)rint((double)v.y * hm);
-    for (int f = f0; f < f1; ++f) {
-      const int pos = s_pos[f];
-      const int c = cb[f] - cbase + (int)rec_field<FMT>(w, pos >> 8, pos & 0xff);
-      __hip_atomic_fetch_add(&lds64[2 * c], gi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      __hip_atomic_fetch_add(&lds64[2 * c + 1], hi_, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  for (int64_t r0 = lo + tid; r0 < hi; r0 += RU * HIST_THREADS) {
+    uint32_t w[RU][U];
+    float2 v[RU];
+#pragma unroll
+    for (int u = 0; u < RU; ++u) {
+      const int64_t r = min(r0 + u * HIST_THREADS, hi - 1);
+      rec_load<FMT>(rec, rb + r, w[u]);
+      v[u] = gh[r];
+    }
+#pragma unroll
+    for (int u = 0; u < RU; ++u) {
+      if (r0 + u * HIST_THREADS >= hi) continue;
+      const unsigned long long gi = (unsigned long long)(long long)rint((double)v[u].x * gm);
+      const unsigned long long hi_ = (unsigned long long)(long long)rint((double)v[u].y * hm);
+#pragma unroll
+      for (int f = 0; f < NS; ++f) {
+        if (f >= f0 && f < f1) {  // uniform
+          const int c = cbr[f] + (int)((w[u][f / BPW] >> (BB * (f % BPW))) & BM);
+          __hip_atomic_fetch_add(&lds64[2 * c], gi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          __hip_atomic_fetch_add(&lds64[2 * c + 1], hi_, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+      }
     }
   }
   __syncthreads();
-  int64_t* out = L.hist_part64 + ((size_t)a * cells + cbase) * 2;
-  for (int c = tid; c < 2 * gcells; c += HIST_THREADS) out[c] = (int64_t)lds64[c];
+  const bool root = (J._pad & 1) != 0;
+  if (root || s_nb[j] <= HIST_FP_SLOTS) {
+    ulonglong2* out = (ulonglong2*)(L.hist_part64 + ((size_t)a * cells + cbase) * 2);
+    for (int c = tid; c < gcells; c += HIST_THREADS) out[c] = ((const ulonglong2*)lds64)[c];
+  } else {
+    unsigned long long* acc = (unsigned long long*)L.hist_acc64 + ((size_t)j * L.acc_cells + cbase) * 2;
+    for (int c = tid; c < 2 * gcells; c += HIST_THREADS)
+      if (lds64[c] != 0ull)
+        __hip_atomic_fetch_add(&acc[c], lds64[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
 }
 
 // ===========================================================================
@@ -733,8 +802,8 @@ __global__ __launch_bounds__(HIST_THREADS) void k_hist_f32(DevLearner L) {
 //                   (exact, from the integer totals), FixHistogram, compaction, and
 //                   the root's FindBestThreshold (wave 0).
 //   mode 2 (build): per-op build into `explicit_out` (no scan).
-// The integer cells are the sum of histogram job 0's partial slots (the wide layout's
-// per-chunk slots); the wide layout's root sums come from its totals cell (its
+// The integer cells are the sum of histogram job 0's partial slots (k_hist_reduce's, or
+// the wide layout's per-chunk slots); the wide layout's root sums come from its totals cell (its
 // most-frequent-bin cells are not accumulated).
 // ===========================================================================
 __global__ __launch_bounds__(SCAN_THREADS) void k_fixscan(DevLearner L, int32_t mode,
@@ -764,7 +833,8 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_fixscan(DevLearner L, int32_t 
           H += (long long)wp[1];
         }
       } else {
-        hist_part_sum64(L, a0, na, ci, &G, &H);
+        G = L.hist_sum64[2 * ci];
+        H = L.hist_sum64[2 * ci + 1];
       }
       if (mode == 1) {
         int64_t* ps = L.int_slots64 + ci * 2;  // node slot 0
@@ -1124,13 +1194,15 @@ int fixscan_prepare() {
   return hipFuncSetAttribute((const void*)k_fixscan, hipFuncAttributeMaxDynamicSharedMemorySize,
                              2 * WIDE_MAX_BIN * (int)sizeof(double)) != hipSuccess;
 }
-void launch_fixscan(const DevLearner& L, int32_t mode, double* explicit_out, hipStream_t s,
+void launch_fixscan(const DevLearner& L, int fp, int32_t mode, double* explicit_out, hipStream_t s,
                     const KernelEvents* ev) {
-  // quantized: the partial slots summed into hist_sum first (f32 cells are summed by
-  // k_fixscan itself); f32 mode never reads hist_sum, so the launch is harmless
-  const int64_t cols = (int64_t)L.total_cells * 3;
-  if (!rec_wide(L.fmt))
-    k_hist_reduce<<<dim3((unsigned)((cols + 15) / 16)), dim3(256), 0, s>>>(L);
+  // the record layouts' partial slots, summed first
+  const int64_t cols = (int64_t)L.total_cells * (fp ? 2 : 3);
+  const dim3 rg((unsigned)((cols + 15) / 16)), rb(256);
+  if (!rec_wide(L.fmt) && fp)
+    k_hist_reduce64<<<rg, rb, 0, s>>>(L);
+  else if (!rec_wide(L.fmt))
+    k_hist_reduce<<<rg, rb, 0, s>>>(L);
   KLAUNCH(ev, k_fixscan, dim3((unsigned)L.F), dim3(SCAN_THREADS),
           (size_t)2 * std::max(L.max_bins, 1) * sizeof(double), s, L, mode, explicit_out);
 }

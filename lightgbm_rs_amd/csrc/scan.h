@@ -901,48 +901,28 @@ __device__ __forceinline__ void lds_hist_flush_clear(unsigned long long* lds, in
   }
 }
 
-// Integer cells (sum q_g, sum q_h, #q_h==3) of cell ci of a histogram job: the sum
-// of its partial slots [a0, a0 + na), four slots per step with independent loads.
-__device__ __forceinline__ void hist_part_sum(const DevLearner& L, int32_t a0, int32_t na, size_t ci,
-                                              int32_t* G, int32_t* H, int32_t* T) {
-  const size_t stride = (size_t)L.total_cells * 3;
-  const int32_t* p = L.hist_part + (size_t)a0 * stride + ci * 3;
-  int32_t g = 0, h = 0, t = 0;
-  int32_t k = 0;
-  for (; k + 4 <= na; k += 4, p += 4 * stride) {
-    int32_t x[12];
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      x[3 * u] = p[u * stride];
-      x[3 * u + 1] = p[u * stride + 1];
-      x[3 * u + 2] = p[u * stride + 2];
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      g += x[3 * u];
-      h += x[3 * u + 1];
-      t += x[3 * u + 2];
-    }
-  }
-  for (; k < na; ++k, p += stride) {
-    g += p[0];
-    h += p[1];
-    t += p[2];
-  }
-  *G = g;
-  *H = h;
-  *T = t;
-}
-
-// The 64-bit fixed-point (g, h) cells of a histogram job (f32 gradients).
-__device__ __forceinline__ void hist_part_sum64(const DevLearner& L, int32_t a0, int32_t na,
-                                                size_t ci, long long* G, long long* H) {
-  const size_t stride = (size_t)L.total_cells * 2;
-  const int64_t* p = L.hist_part64 + (size_t)a0 * stride + ci * 2;
+// The 64-bit fixed-point (g, h) cells of a child job (f32 gradients): the sum of its
+// slots, all loads in flight, or its accumulator, which is cleared.
+__device__ __forceinline__ void hist_child_sum64(const DevLearner& L, int32_t j, int32_t a0,
+                                                 int32_t na, size_t ci, long long* G, long long* H) {
   long long g = 0, h = 0;
-  for (int32_t k = 0; k < na; ++k, p += stride) {
-    g += p[0];
-    h += p[1];
+  if (na > HIST_FP_SLOTS) {
+    longlong2* acc = (longlong2*)L.hist_acc64 + (size_t)j * L.acc_cells + ci;
+    const longlong2 x = *acc;
+    *acc = make_longlong2(0, 0);
+    g = x.x;
+    h = x.y;
+  } else {
+    const longlong2* p = (const longlong2*)L.hist_part64 + (size_t)a0 * L.total_cells + ci;
+    longlong2 x[HIST_FP_SLOTS];
+#pragma unroll
+    for (int k = 0; k < HIST_FP_SLOTS; ++k)
+      x[k] = k < na ? p[(size_t)k * L.total_cells] : make_longlong2(0, 0);
+#pragma unroll
+    for (int k = 0; k < HIST_FP_SLOTS; ++k) {
+      g += x[k].x;
+      h += x[k].y;
+    }
   }
   *G = g;
   *H = h;
