@@ -178,6 +178,7 @@ struct lgbm_hip_ctx {
   bool no_bincol = false;   // LGBM_HIP_BINCOL=0: the wide layout without its feature-major copy
   int32_t max_bins = 0;     // the widest feature's num_bin
   int32_t has_cat = 0;      // some feature is categorical
+  int32_t scan_wide = 0;    // the child scans take k_pair_scan_wide
   bool bin16 = false;       // wide layout with 2-byte bins
   int32_t n_wgroups = 0;    // 2-byte bins: feature groups of the histogram kernel
   int32_t* d_wgroups = nullptr;  // [n_wgroups + 1] first feature of each group
@@ -448,6 +449,7 @@ DevLearner make_learner(lgbm_hip_ctx* c) {
   L.row_stride = c->row_stride;
   L.max_bins = c->max_bins;
   L.has_cat = c->has_cat;
+  L.scan_wide = c->scan_wide;
   L.bin16 = c->bin16 ? 1 : 0;
   L.n_wgroups = c->n_wgroups;
   L.wgroups = c->d_wgroups;
@@ -1168,6 +1170,9 @@ int resident_setup(lgbm_hip_ctx* c, int32_t F_in, int64_t num_data, const lgbm_f
   c->has_cat = 0;
   for (int f = 0; f < F; ++f)
     if (meta[f].bin_type == LGBM_BIN_CATEGORICAL) c->has_cat = 1;
+  c->scan_wide = wide && !bin16 && !c->has_cat ? 1 : 0;
+  for (const DevFeature& d : feats)
+    if (d.run_forward || d.skip_default_bin || d.na_as_missing) c->scan_wide = 0;
   c->bin16 = bin16;
   c->fmt = (F + 4 + 15) / 16;
   if (wide) {

@@ -1548,6 +1548,314 @@ __global__ __launch_bounds__(SCAN_THREADS, 6) void k_pair_scan(DevLearner L, int
 }
 
 // ===========================================================================
+// k_pair_scan_wide: k_pair_scan for the wide layout's rounds, whose F x jobs scans are more
+// than the chip holds, so that their VALU work sets the round's time.  The reference's
+// FixHistogram chain and threshold prefix are sequential f64 sums; one wave per (feature,
+// child) runs such a sum with all 64 lanes on the same 256 steps.  Here a block of four
+// waves takes PSW_F features of a job, and a lane runs one component (gradient or hessian)
+// of one feature's and child's sum, in the reference's order, in LDS; then the waves
+// evaluate the candidates, 64 a step.  Raw bins are indexed throughout (compaction only
+// shifts them).  For datasets without missing values, categorical features and 2-byte
+// bins; the others keep k_pair_scan.
+//
+// 2M rows x 700 features, quantized, 255 leaves: 41 -> 36 us a round; 1M x 2000, f32: 43 ->
+// 35 (four features a block 45 and 37, eight slower still: a block's sums are a serial
+// chain, which more blocks beside it hide).  What is left is the candidates' f64 divisions
+// and the chain.
+// ===========================================================================
+constexpr int PSW_F = 2;         // features a block
+constexpr int PSW_THREADS = 256;
+constexpr int PSW_BATCHES = 4;   // 64-candidate batches of at most 256 bins
+constexpr int PSW_AHEAD = 8;     // steps of a sum whose cells are loaded ahead
+// cells of a row: the bins, the spare cells that a sum's last steps and loads overrun into on
+// either side (the row before's on the low side), and one that spreads the rows over the banks
+__host__ __device__ constexpr int psw_row(int max_bins) { return max_bins + 2 * PSW_AHEAD + 1; }
+template <bool FP>
+__global__ __launch_bounds__(PSW_THREADS, 4) void k_pair_scan_wide(DevLearner L) {
+  extern __shared__ __align__(16) double2 psw_all[];  // [PSW_F][smaller, larger][row]
+  __shared__ DevFeature s_ft[PSW_F];
+  __shared__ double2 s_pm[PSW_F];
+  __shared__ int32_t s_on[PSW_F];
+  Ctl* ctl = L.ctl;
+  const int j = blockIdx.y, tid = threadIdx.x, F = L.F, cells = L.total_cells;
+  const int f0 = (int)blockIdx.x * PSW_F, nf = min(PSW_F, F - f0);
+  const int row = psw_row(L.max_bins);
+  double2* psw_lds = psw_all + 2 * PSW_AHEAD;  // bin 0 of the first row
+  const int32_t n_jobs = ctl->n_jobs;
+  const PartJob& J = ctl->jobs[j];  // slot j always exists; its fields are used below
+  const int32_t p = J.parent, cl = J.cl, cr = J.cr, acc_right = J.acc_right;
+  const int32_t a0 = ctl->hjobs[j].a0, na = ctl->hjobs[j].nblk;
+  const int32_t md = ctl->max_depth, min2 = ctl->cfg.min_data_in_leaf * 2;
+  const ScanCfg sc = make_scan_cfg(ctl->cfg);
+  if (j >= n_jobs) return;
+  const DevNodes& nd = L.nodes;
+  const int32_t lcnt = nd.count[cl], rcnt = nd.count[cr], dcl = nd.depth[cl];
+  const LeafSums scl = nd.sums[cl], scr = nd.sums[cr];
+  const bool pmat = L.fmat[p] != 0;
+  const bool gated = (md > 0 && dcl >= md) || (lcnt < min2 && rcnt < min2);
+  const bool right_small = !(lcnt < rcnt);
+  const int32_t sm = right_small ? cr : cl, lg = right_small ? cl : cr;
+  const LeafSums ss = right_small ? scr : scl, gs = right_small ? scl : scr;
+  const bool sm_zero = !(ss.sh > 0.0 && ss.n > 0);
+  const bool lg_mat = pmat || sm_zero;  // (k_pair_scan)
+  if (blockIdx.x == 0 && tid == 0) {
+    L.fmat[sm] = 0;
+    L.fmat[lg] = lg_mat ? 1 : 0;
+  }
+  if (tid < nf) {
+    const int f = f0 + tid;
+    const bool on = L.splittable[(size_t)p * F + f] != 0;
+    s_ft[tid] = L.feats[f];
+    s_pm[tid] = L.mfbv[(size_t)p * F + f];
+    s_on[tid] = on ? 1 : 0;
+    if (gated || !on) {
+      // no scan (k_pair_scan): a parent that cannot split on the feature passes that on
+      split_set_none(&L.feat_split[(size_t)sm * F + f]);
+      split_set_none(&L.feat_split[(size_t)lg * F + f]);
+      L.gain_dense[(size_t)sm * F + f] = -__builtin_inf();
+      L.gain_dense[(size_t)lg * F + f] = -__builtin_inf();
+      if (!gated && !sm_zero) L.splittable[(size_t)sm * F + f] = 0;
+      if (!gated && gs.sh > 0.0 && gs.n > 0) L.splittable[(size_t)lg * F + f] = 0;
+    }
+  } else if (tid < PSW_F) {
+    s_on[tid] = 0;
+    s_ft[tid] = DevFeature{};
+  }
+  if (gated) return;
+  __syncthreads();
+  // ---- cells: the built side from its chunks, the other side = parent - built ---------
+  const double vg1 = (double)ctl->vg1, vh1 = (double)ctl->vh1, vh3 = (double)ctl->vh3;
+  const double gu = FP ? ldexp(1.0, -ctl->g_shift) : 0.0, hu = FP ? ldexp(1.0, -ctl->h_shift) : 0.0;
+  const int b = tid;  // at most 256 bins: one a thread
+  if constexpr (FP) {
+    longlong2 S[PSW_F], P[PSW_F];
+#pragma unroll
+    for (int q = 0; q < PSW_F; ++q) {
+      const bool in = s_on[q] && b < (int)s_ft[q].num_bin;
+      S[q] = make_longlong2(0, 0);
+      P[q] = in ? ((const longlong2*)L.int_slots64)[(size_t)p * cells + s_ft[q].cell_base + b]
+                : make_longlong2(0, 0);
+    }
+    const longlong2* wp = (const longlong2*)L.wide_part + (size_t)a0 * cells + b;
+    for (int k0 = 0; k0 < na; k0 += 2) {
+      longlong2 x[2][PSW_F];
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int q = 0; q < PSW_F; ++q) {
+          const bool in = k0 + u < na && s_on[q] && b < (int)s_ft[q].num_bin;
+          x[u][q] = in ? wp[(size_t)(k0 + u) * cells + s_ft[q].cell_base] : make_longlong2(0, 0);
+        }
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int q = 0; q < PSW_F; ++q) {
+          S[q].x += x[u][q].x;
+          S[q].y += x[u][q].y;
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < PSW_F; ++q) {
+      if (!s_on[q] || b >= (int)s_ft[q].num_bin) continue;
+      const size_t ci = s_ft[q].cell_base + b;
+      const longlong2 O = make_longlong2(P[q].x - S[q].x, P[q].y - S[q].y);
+      ((longlong2*)L.int_slots64)[(size_t)sm * cells + ci] = S[q];
+      ((longlong2*)L.int_slots64)[(size_t)lg * cells + ci] = O;
+      double2* c = psw_lds + (size_t)(2 * q) * row;
+      c[b] = sm_zero ? make_double2(0.0, 0.0) : make_double2((double)S[q].x * gu, (double)S[q].y * hu);
+      c[row + b] = make_double2((double)(lg_mat ? P[q].x : O.x) * gu,
+                                (double)(lg_mat ? P[q].y : O.y) * hu);
+    }
+  } else {
+    int32_t A[PSW_F][3], P[PSW_F][3];
+#pragma unroll
+    for (int q = 0; q < PSW_F; ++q) {
+      const bool in = s_on[q] && b < (int)s_ft[q].num_bin;
+      const int32_t* ps = L.int_slots + ((size_t)p * cells + s_ft[q].cell_base + (in ? b : 0)) * 3;
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        A[q][i] = 0;
+        P[q][i] = in ? ps[i] : 0;
+      }
+    }
+    const unsigned long long* wp = L.wide_part + (size_t)a0 * cells + b;
+    for (int k0 = 0; k0 < na; k0 += 4) {
+      unsigned long long x[4][PSW_F];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int q = 0; q < PSW_F; ++q) {
+          const bool in = k0 + u < na && s_on[q] && b < (int)s_ft[q].num_bin;
+          x[u][q] = in ? wp[(size_t)(k0 + u) * cells + s_ft[q].cell_base] : 0ull;
+        }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int q = 0; q < PSW_F; ++q) {
+          int32_t g_, h_, t_;
+          unpack_cell(x[u][q], &g_, &h_, &t_);
+          A[q][0] += g_;
+          A[q][1] += h_;
+          A[q][2] += t_;
+        }
+    }
+    const int32_t bs = acc_right ? cr : cl, os = acc_right ? cl : cr;  // built, other side
+#pragma unroll
+    for (int q = 0; q < PSW_F; ++q) {
+      if (!s_on[q] || b >= (int)s_ft[q].num_bin) continue;
+      const size_t ci = s_ft[q].cell_base + b;
+      int32_t O[3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        O[i] = P[q][i] - A[q][i];
+        L.int_slots[((size_t)bs * cells + ci) * 3 + i] = A[q][i];
+        L.int_slots[((size_t)os * cells + ci) * 3 + i] = O[i];
+      }
+      const bool small_built = sm == bs;
+      double2* c = psw_lds + (size_t)(2 * q) * row;
+      double2 vs, vl;
+      int_cell_to_f64(small_built ? A[q][0] : O[0], small_built ? A[q][1] : O[1],
+                      small_built ? A[q][2] : O[2], vg1, vh1, vh3, &vs.x, &vs.y);
+      int_cell_to_f64(lg_mat ? P[q][0] : small_built ? O[0] : A[q][0],
+                      lg_mat ? P[q][1] : small_built ? O[1] : A[q][1],
+                      lg_mat ? P[q][2] : small_built ? O[2] : A[q][2], vg1, vh1, vh3, &vl.x, &vl.y);
+      c[b] = sm_zero ? make_double2(0.0, 0.0) : vs;
+      c[row + b] = vl;
+    }
+  }
+  constexpr int U = PSW_AHEAD;
+  // the smaller child's spare cells, which the chain below overruns into: x - (+0.0) == x
+  if (tid < PSW_F * 2 * U)
+    psw_lds[(size_t)(2 * (tid / (2 * U))) * row + (int)s_ft[tid / (2 * U)].num_bin + tid % (2 * U)] =
+        make_double2(0.0, 0.0);
+  __syncthreads();
+  // ---- FixHistogram of the smaller child; the larger's fixed cell (fix_compact_pair) ----
+  if (tid < 2 * PSW_F) {
+    const int q = tid >> 1, comp = tid & 1;
+    const int nb = (int)s_ft[q].num_bin, mfb = (int)s_ft[q].mfb;
+    if (s_on[q] && mfb > 0 && mfb < nb) {
+      double* c = (double*)(psw_lds + (size_t)(2 * q) * row) + comp;
+      double x = 0.0;
+      if (!sm_zero) {
+        c[2 * mfb] = 0.0;
+        x = comp ? ss.sh : ss.sg;
+        double v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = c[2 * u];
+        for (int i0 = U; i0 < nb + U; i0 += U) {  // the next cells load while these are taken off
+          double w[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) w[u] = c[2 * (i0 + u)];
+#pragma unroll
+          for (int u = 0; u < U; ++u) x -= v[u];
+#pragma unroll
+          for (int u = 0; u < U; ++u) v[u] = w[u];
+        }
+        c[2 * mfb] = x;
+      }
+      const double pm = comp ? s_pm[q].y : s_pm[q].x;
+      c[2 * (row + mfb)] = lg_mat ? pm : pm - x;
+    }
+  }
+  __syncthreads();
+  const size_t sl = L.slot_len;
+  if (lg_mat) {
+    // larger = parent - smaller cell by cell, kept (compacted) in the node's f64 slot
+    for (int q = 0; q < PSW_F; ++q) {
+      const int nb = (int)s_ft[q].num_bin, off = s_ft[q].offset;
+      if (!s_on[q] || b >= nb) continue;
+      double2* c = psw_lds + (size_t)(2 * q) * row;
+      const double2* par = (const double2*)(L.slots + (size_t)p * sl + s_ft[q].slot_off);
+      double2* out = (double2*)(L.slots + (size_t)lg * sl + s_ft[q].slot_off);
+      if (b >= off) {
+        const double2 P = pmat ? par[b - off] : c[row + b];
+        const double2 d = make_double2(P.x - c[b].x, P.y - c[b].y);
+        c[row + b] = d;
+        out[b - off] = d;
+      } else {
+        out[nb - 1] = make_double2(0.0, 0.0);  // zeros enter at the top
+      }
+    }
+    __syncthreads();
+  }
+  if (tid < nf && s_on[tid]) {
+    const int mfb = (int)s_ft[tid].mfb;
+    if (mfb > 0 && mfb < (int)s_ft[tid].num_bin) {
+      const double2* c = psw_lds + (size_t)(2 * tid) * row + mfb;
+      L.mfbv[(size_t)sm * F + f0 + tid] = c[0];
+      L.mfbv[(size_t)lg * F + f0 + tid] = c[row];
+    }
+  }
+  // ---- row counts of the candidates, before the sums take the cells' place --------------
+  constexpr int kPairs = 2 * PSW_F / (PSW_THREADS / LGBM_WAVE);  // (feature, child) a wave
+  const int lane = (int)lane_id(), wave = tid >> 6;
+  int32_t cnt[kPairs][PSW_BATCHES];
+#pragma unroll
+  for (int i = 0; i < kPairs; ++i) {
+    const int pair = wave * kPairs + i, q = pair >> 1;
+    const LeafSums& ls = (pair & 1) ? gs : ss;
+    const double cf = (double)ls.n / (ls.sh + 2.0 * k_eps());
+    const int nb = s_on[q] ? (int)s_ft[q].num_bin : 0;
+#pragma unroll
+    for (int k = 0; k < PSW_BATCHES; ++k) {
+      const int r = nb - 1 - k * LGBM_WAVE - lane;
+      cnt[i][k] = r >= 1 ? round_int(psw_lds[(size_t)pair * row + r].y * cf) : 0;
+    }
+  }
+  __syncthreads();
+  // ---- prefix sums from the top bin down, from kEpsilon (split.rs:9078-9176) -------------
+  if (tid < 4 * PSW_F) {
+    const int pair = tid >> 1, comp = tid & 1, q = pair >> 1;
+    const int nb = s_on[q] ? (int)s_ft[q].num_bin : 0;
+    double* c = (double*)(psw_lds + (size_t)pair * row) + comp;
+    double x = comp ? k_eps() : 0.0;
+    double v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = c[2 * (nb - 1 - u)];
+    for (int r0 = nb - 1; r0 >= 1; r0 -= U) {
+      double w[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) w[u] = c[2 * (r0 - U - u)];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        x += v[u];
+        v[u] = x;
+      }
+      // the last steps write bin 0, which no candidate reads, and spare cells
+#pragma unroll
+      for (int u = 0; u < U; ++u) c[2 * (r0 - u)] = v[u];
+#pragma unroll
+      for (int u = 0; u < U; ++u) v[u] = w[u];
+    }
+  }
+  __syncthreads();
+  // ---- candidates ---------------------------------------------------------------------
+#pragma unroll
+  for (int i = 0; i < kPairs; ++i) {
+    const int pair = wave * kPairs + i, q = pair >> 1;
+    if (!s_on[q]) continue;
+    const int32_t leaf = (pair & 1) ? lg : sm;
+    const LeafSums& ls = (pair & 1) ? gs : ss;
+    lgbm_split_info* out = L.feat_split + (size_t)leaf * F + f0 + q;
+    double* out_gain = L.gain_dense + (size_t)leaf * F + f0 + q;
+    if (!(ls.sh > 0.0 && ls.n > 0)) {
+      if (lane == 0) {
+        split_set_none(out);
+        *out_gain = -__builtin_inf();
+      }
+      continue;
+    }
+    const double gain = wave_scan_sums(psw_lds + (size_t)pair * row, cnt[i], (int)s_ft[q].num_bin,
+                                       sc, ls.sg, ls.sh, ls.n, ls.weight, out);
+    if (lane == 0) {
+      L.splittable[(size_t)leaf * F + f0 + q] = gain > -__builtin_inf() ? 1 : 0;
+      out->gain = gain * s_ft[q].penalty;
+      *out_gain = gain * s_ft[q].penalty;
+    }
+  }
+}
+
+// ===========================================================================
 // k_tree_finalize: the Tree's leaf arrays from the committed leaves' node slots
 // (leaf_value = the leaf's output, leaf_weight = its sum_hessian, 0 for an unsplit
 // root: Tree::root, learner.rs:5398-5424), its linkage and real thresholds, the
@@ -1784,6 +2092,16 @@ int scan_prepare() {
 
 void launch_pair_scan(const DevLearner& L, int fp, int32_t spec_max, int32_t part_grid,
                       hipStream_t s, const KernelEvents* ev) {
+  if (L.scan_wide) {
+    const size_t rows =
+        ((size_t)2 * PSW_F * psw_row(L.max_bins) + 2 * PSW_AHEAD) * sizeof(double2);
+    const dim3 gw((unsigned)((L.F + PSW_F - 1) / PSW_F), (unsigned)spec_max), bw(PSW_THREADS);
+    if (fp)
+      KLAUNCH(ev, (k_pair_scan_wide<true>), gw, bw, rows, s, L);
+    else
+      KLAUNCH(ev, (k_pair_scan_wide<false>), gw, bw, rows, s, L);
+    return;
+  }
   const size_t lds = (size_t)4 * std::max(L.max_bins, 1) * sizeof(double);
   const dim3 g((unsigned)L.F, (unsigned)spec_max), b(SCAN_THREADS);
   // quantized cells are exact unit multiples while every sum stays below 2^53 units

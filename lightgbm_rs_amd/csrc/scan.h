@@ -458,6 +458,94 @@ __device__ __attribute__((unused)) double wave_scan(const double* hist, const De
   return any_split && best_gain > ninf ? best_gain - mgs : ninf;
 }
 
+// wave_scan of a feature without missing values whose REVERSE prefix sums are already
+// there: P[r] holds the sums over bins r .. num_bin - 1 (raw bins, from kEpsilon on, in the
+// reference's order) and cnt[k] this lane's row count of bin num_bin - 1 - 64 k - lane.
+// Such a feature has no FORWARD scan (split.rs:9178).
+template <int NB>
+__device__ __forceinline__ double wave_scan_sums(const double2* P, const int32_t (&cnt)[NB],
+                                                 int32_t nb, const ScanCfg& c,
+                                                 double sum_gradient, double sum_hessian,
+                                                 int32_t num_data, double po,
+                                                 lgbm_split_info* out) {
+  const int lane = (int)lane_id();
+  const double eps = k_eps();
+  const double ninf = -__builtin_inf();
+  const double shb = sum_hessian + 2.0 * eps;
+  const double gain_shift =
+      c.use_full ? leaf_gain_full(c.use_l1, sum_gradient, shb, c.l1, c.l2, c.mds, c.use_smoothing,
+                                  c.ps, num_data, po)
+                 : leaf_gain(c.use_l1, sum_gradient, shb, c.l1, c.l2);
+  const double mgs = gain_shift + c.min_gain;
+  // each lane's best candidate so far (its first, being replaced by larger gains only)
+  double my_gain = ninf;
+  int32_t my_at = 0, my_lc = 0, cc = 0;
+  const int32_t rev_count = max(nb - 1, 0);
+#pragma unroll
+  for (int k = 0; k < NB; ++k) {
+    const int32_t base = k * LGBM_WAVE;
+    if (base >= rev_count) break;
+    const int32_t n = min(LGBM_WAVE, rev_count - base);
+    const int32_t r = nb - 1 - base - lane;
+    const bool act = lane < n;
+    const double2 s = act ? P[r] : make_double2(0.0, 0.0);
+    const double sg = s.x, sh = s.y;
+    const int32_t rc = cc + wave_incl_sum_i32(act ? cnt[k] : 0);
+    const int32_t lc = num_data - rc;
+    const double slh = shb - sh, slg = sum_gradient - sg;
+    const bool cont = rc < c.min_d || sh < c.min_h;
+    const bool brk = lc < c.min_d || slh < c.min_h;
+    const unsigned long long bm = __ballot(act && !cont && brk);
+    const int first_brk = bm ? (__ffsll((unsigned long long)bm) - 1) : LGBM_WAVE;
+    if (act && !cont && lane < first_brk) {
+      const double gain = split_gain_of(c, slg, slh, sg, sh, lc, rc, po);
+      if (gain > mgs && gain > my_gain) {
+        my_gain = gain;
+        my_at = base + lane;
+        my_lc = lc;
+      }
+    }
+    if (bm) break;
+    cc = readlane_i32(rc, n - 1);
+  }
+  // the highest gain, the first candidate among equal ones
+  const double best_gain = wave_max_f64(my_gain);
+  const bool any_split = best_gain > ninf;
+  unsigned long long tie = __ballot(any_split && my_gain == best_gain);
+  int rl = tie ? (int)__builtin_ctzll(tie) : 0;
+  for (tie &= tie - 1; tie; tie &= tie - 1) {
+    const int o = (int)__builtin_ctzll(tie);
+    if (readlane_i32(my_at, o) < readlane_i32(my_at, rl)) rl = o;
+  }
+  const int32_t at = readlane_i32(my_at, rl), best_lc = readlane_i32(my_lc, rl);
+  const int32_t best_thr = nb - 2 - at;
+  const double2 bs = any_split ? P[nb - 1 - at] : make_double2(0.0, 0.0);
+  const double best_lg = sum_gradient - bs.x, best_lh = shb - bs.y;
+  if (lane == 0) {
+    if (any_split && best_gain > ninf) {
+      const int32_t best_rc = num_data - best_lc;
+      const double rsg = sum_gradient - best_lg;
+      const double rsh = shb - best_lh;
+      out->threshold = (uint32_t)best_thr;
+      out->gain = best_gain - mgs;
+      out->left_count = best_lc;
+      out->right_count = best_rc;
+      out->left_sum_gradient = best_lg;
+      out->left_sum_hessian = best_lh - eps;
+      out->right_sum_gradient = rsg;
+      out->right_sum_hessian = rsh - eps;
+      out->left_output = leaf_output_full(c.use_l1, best_lg, best_lh, c.l1, c.l2, c.mds,
+                                          c.use_smoothing, c.ps, best_lc, po);
+      out->right_output = leaf_output_full(c.use_l1, rsg, rsh, c.l1, c.l2, c.mds,
+                                           c.use_smoothing, c.ps, best_rc, po);
+      out->default_left = 1;
+    } else {
+      split_set_none(out);
+    }
+  }
+  return any_split && best_gain > ninf ? best_gain - mgs : ninf;
+}
+
 // ===========================================================================
 // FindBestThresholdCategorical for one (leaf, feature) by one wave
 // (feature_histogram_categorical.rs:96-495) over the compacted histogram (index t =
