@@ -46,14 +46,17 @@
 #ifndef WIDE_THREADS
 #define WIDE_THREADS 1024
 #endif
-// row-chunk blocks over all groups (at least), per gradient mode: more chunks spread
-// the large builds over more blocks, fewer leave the scans fewer partial slots to sum
-#ifndef WIDE_GRID_Q
-#define WIDE_GRID_Q 512                 // quantized: 64-feature groups, 8-byte cells
-#endif
-#ifndef WIDE_GRID_F
-#define WIDE_GRID_F 1024                // f32: 32-feature groups, 16-byte cells
-#endif
+// row-chunk blocks over all groups: one a CU, whose 128 KiB of LDS a block fills.  A chunk's
+// cost is its cells' stores and the scans' loads of them, not its rows' adds (leaving a fifth
+// of the adds out measured no gain), so fewer, longer chunks are faster: 1M x 2000, f32, ten
+// trees of 127 leaves, 1024 / 512 / 256 blocks 76.2 / 74.7 / 73.3 ms; 2M x 100 x 10 classes
+// 48.1 / 47.3 / 47.6; 2M x 700 quantized, ten trees of 255 leaves, 512 / 256 / 128 blocks
+// 94.1 / 93.3 / 98.0.  Past WIDE_GRID_GROUPS groups, whole chunks of all groups leave up to a
+// third of the CUs without a block, and the larger grids stay.
+#define WIDE_GRID 256
+#define WIDE_GRID_GROUPS 64
+#define WIDE_GRID_MANY_Q 512
+#define WIDE_GRID_MANY_F 1024
 #ifndef WIDE_MIN_ROWS
 #define WIDE_MIN_ROWS 4096              // rows per chunk (at least): a flush costs a group
 #endif

@@ -464,7 +464,8 @@ int wide_groups(int32_t F, int fp, int32_t n_groups16) {
 // Blocks per feature group of a launch (row chunks + one per job at most): rows per
 // chunk stay <= WIDE_MAX_ROWS, and the grid fills the chip.
 int64_t wide_grid_x(int ng, int64_t N, int fp) {
-  int64_t chunks = std::max<int64_t>((fp ? WIDE_GRID_F : WIDE_GRID_Q) / ng,
+  const int grid = ng <= WIDE_GRID_GROUPS ? WIDE_GRID : fp ? WIDE_GRID_MANY_F : WIDE_GRID_MANY_Q;
+  int64_t chunks = std::max<int64_t>(grid / ng,
                                      (N + WIDE_MAX_ROWS - 1) / WIDE_MAX_ROWS);
   return std::max<int64_t>(chunks, 1) + SPEC_MAX;
 }
