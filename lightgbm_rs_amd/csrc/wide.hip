@@ -66,6 +66,11 @@ __global__ __launch_bounds__(WIDE_THREADS) void k_hist_wide(DevLearner L) {
   constexpr int NV = GF / 16;      // 16-byte words of a row's group bytes
   constexpr int RU = FP ? 4 : 2;   // rows per thread in flight
   constexpr int NW = WIDE_THREADS / LGBM_WAVE;
+  // f32: gradients' cells from 0, hessians' from H0.  Side by side, either sum's cells would
+  // be 16 bytes apart and its adds use half of the banks: 2M rows x 100 dense columns, ten
+  // trees of 127 leaves, 48.2 -> 45.0 ms; 1M x 2000 of 90 % zeros, few lanes an add, 73.4 and
+  // 73.6.
+  constexpr int H0 = B16 ? WIDE16_GROUP_CELLS : GF * 256;
   extern __shared__ unsigned long long lds[];
   __shared__ uint32_t s_fd[GF];    // per feature: (first cell - group base) << 8 | mfb
                                    // (2-byte bins: << 16)
@@ -109,7 +114,10 @@ __global__ __launch_bounds__(WIDE_THREADS) void k_hist_wide(DevLearner L) {
     }
     s_fd[k] = d;
   }
-  for (int c = tid; c < gcells * (FP ? 2 : 1); c += WIDE_THREADS) lds[c] = 0ull;
+  for (int c = tid; c < gcells; c += WIDE_THREADS) {
+    lds[c] = 0ull;
+    if constexpr (FP) lds[H0 + c] = 0ull;
+  }
   __syncthreads();
 
   const HistJob& J = ctl->hjobs[j];
@@ -157,9 +165,9 @@ __global__ __launch_bounds__(WIDE_THREADS) void k_hist_wide(DevLearner L) {
           const uint32_t fd = __builtin_amdgcn_readfirstlane(s_fd[k0 + k]);
           if (bins[k] != (fd & 0xffu)) {
             const int c = (int)(fd >> 8) + (int)bins[k];
-            __hip_atomic_fetch_add(&lds[2 * c], (unsigned long long)gi, __ATOMIC_RELAXED,
+            __hip_atomic_fetch_add(&lds[c], (unsigned long long)gi, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_WORKGROUP);
-            __hip_atomic_fetch_add(&lds[2 * c + 1], (unsigned long long)hi_, __ATOMIC_RELAXED,
+            __hip_atomic_fetch_add(&lds[H0 + c], (unsigned long long)hi_, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_WORKGROUP);
           }
         }
@@ -288,8 +296,8 @@ __global__ __launch_bounds__(WIDE_THREADS) void k_hist_wide(DevLearner L) {
           if (bin != (d & 0xffffu)) {
             const int c = (int)(d >> 16) + (int)bin;
             if constexpr (FP) {
-              __hip_atomic_fetch_add(&lds[2 * c], va[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-              __hip_atomic_fetch_add(&lds[2 * c + 1], vb[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+              __hip_atomic_fetch_add(&lds[c], va[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+              __hip_atomic_fetch_add(&lds[H0 + c], vb[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             } else {
               __hip_atomic_fetch_add(&lds[c], va[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             }
@@ -314,8 +322,8 @@ __global__ __launch_bounds__(WIDE_THREADS) void k_hist_wide(DevLearner L) {
             if (bin != (fd[k] & 0xffu)) {
               const int c = (int)(fd[k] >> 8) + (int)bin;
               if constexpr (FP) {
-                __hip_atomic_fetch_add(&lds[2 * c], va[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                __hip_atomic_fetch_add(&lds[2 * c + 1], vb[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                __hip_atomic_fetch_add(&lds[c], va[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                __hip_atomic_fetch_add(&lds[H0 + c], vb[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
               } else {
                 __hip_atomic_fetch_add(&lds[c], va[u], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
               }
@@ -330,7 +338,12 @@ __global__ __launch_bounds__(WIDE_THREADS) void k_hist_wide(DevLearner L) {
   {
     constexpr int CW = FP ? 2 : 1;  // u64 words per cell
     unsigned long long* dst = L.wide_part + ((size_t)a * cells + gbase) * CW;
-    for (int c = tid; c < gcells * CW; c += WIDE_THREADS) dst[c] = lds[c];
+    for (int c = tid; c < gcells; c += WIDE_THREADS) {
+      if constexpr (FP)
+        ((ulonglong2*)dst)[c] = make_ulonglong2(lds[c], lds[H0 + c]);
+      else
+        dst[c] = lds[c];
+    }
   }
   if (totals) {
 #pragma unroll
