@@ -10,6 +10,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <string>
 #include <type_traits>
@@ -3370,7 +3371,13 @@ int predict_prepare(lgbm_hip_ctx* c, const lgbm_hip_model* m, int64_t rows, int3
     if ((rc = upload_vec(c, &c->pm_expv, m->tree_expected))) return rc;
     PredPacked pk;
     c->pack = PredPack{};
-    if (model_pack_trees(*m, &pk)) {
+    bool packed = false;
+    try {
+      packed = model_pack_trees(*m, &pk);
+    } catch (const std::exception& e) {  // no host memory: not past the C entry
+      return set_err(c, LGBM_HIP_ERR_RUNTIME, e.what());
+    }
+    if (packed) {
       if (!c->pack_lds && predict_lds_prepare())
         return set_err(c, LGBM_HIP_ERR_HIP, "the prediction kernels' LDS size was refused");
       c->pack_lds = true;
@@ -3498,7 +3505,11 @@ int predict_run(lgbm_hip_ctx* c, const lgbm_hip_model* m, const float* d_x, int6
     if (it0 < it1 && depth <= SHAP_MAX_DEPTH && leaves <= SHAP_MAX_LEAVES &&
         shap_rows_per_block(m->max_feature_idx + 1, leaves) > 0 &&
         m->leaf_values.size() < (size_t)1 << 22)  // feature offsets fit 27 bits
-      return contrib_paths(c, m, d_x, rows, cols, it0, it1, leaves, (double*)d_out);
+      try {
+        return contrib_paths(c, m, d_x, rows, cols, it0, it1, leaves, (double*)d_out);
+      } catch (const std::exception& e) {
+        return set_err(c, LGBM_HIP_ERR_RUNTIME, e.what());
+      }
     // the deepest tree of the range sizes each row's path buffer; rows go in chunks
     // whose workspace stays within 256 MiB
     const int64_t per_row = shap_bytes_per_row(depth);
