@@ -895,6 +895,9 @@ __global__ __launch_bounds__(256) void k_shap_rows(
         }
 #pragma unroll
         for (int u = 0; u < B; ++u) {
+          // a leaf's features are its path's own, but the leaf before may have met one of
+          // them in another lane: its adds come first
+          wave_lds_sync();
           if (f[u] >= 0) phi[f[u]] += c[u];
           for (int i = gl + G; i < (int)(e[u].y & 31u); i += G)
             phi[feats[(e[u].y >> 5) + i]] += tab[e[u].x + i];

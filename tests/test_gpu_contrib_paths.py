@@ -62,3 +62,20 @@ def test_bits_equal_the_recursion(be, leaves, cols, classes, chain):
         X[rng.random(X.shape) < 0.1] = 0.0
         got, ref = be.predict(m, X, "contrib"), P.predict_contrib(pm, X)
         assert np.array_equal(got.view(np.uint64), np.ascontiguousarray(ref).view(np.uint64))
+
+
+# Each leaf of a chain whose nodes take the features in turn has the features of the leaf
+# before it one position (and so one lane of k_shap_rows) further on: every add follows
+# another lane's to the same sum.
+@pytest.mark.parametrize("cols", [2, 3, 8, 9, 16])
+def test_consecutive_leaves_meet_the_same_features(be, cols):
+    rng = np.random.default_rng(cols)
+    m = Model.create(num_class=1, max_feature_idx=cols - 1)
+    for _ in range(3):
+        t = _tree(rng, 30, cols, True)
+        t["split_feature"] = (np.arange(29) % cols).astype(np.int32)
+        m.add_tree(t)
+    print(f"contrib rotating features cols={cols}", flush=True)
+    X = rng.normal(size=(70, cols)).astype(np.float32)
+    got, ref = be.predict(m, X, "contrib"), P.predict_contrib(P.parse_model(m.to_text()), X)
+    assert np.array_equal(got.view(np.uint64), np.ascontiguousarray(ref).view(np.uint64))
