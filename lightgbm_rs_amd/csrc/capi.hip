@@ -3476,6 +3476,15 @@ int contrib_paths(lgbm_hip_ctx* c, const lgbm_hip_model* m, const float* d_x, in
   return LGBM_HIP_OK;
 }
 
+// The call as predict_lds_shape sees it: rows of `cols` columns in memory.
+PredCall predict_call(const lgbm_hip_ctx* c, const lgbm_hip_model* m, int64_t rows, int32_t cols,
+                      int32_t it0, int32_t it1, PredForm form, int64_t nnz = 0) {
+  return PredCall{rows, cols, c->pack.stride,
+                  (it1 - it0) * m->num_tree_per_iteration,
+                  (double)m->leaf_values.size() / (double)std::max<size_t>(m->tree_index.size(), 1),
+                  form, (double)nnz / (double)std::max<int64_t>(rows, 1)};
+}
+
 // Enqueues k_predict_lds over R's rows.
 void predict_lds_run(lgbm_hip_ctx* c, const lgbm_hip_model* m, const PredShape& shape,
                      const PredRows& R, bool csr, int64_t rows, int32_t width, int32_t it0,
@@ -3494,7 +3503,8 @@ void predict_lds_run(lgbm_hip_ctx* c, const lgbm_hip_model* m, const PredShape& 
 
 int predict_run(lgbm_hip_ctx* c, const lgbm_hip_model* m, const float* d_x, int64_t rows,
                 int32_t cols, int32_t it0, int32_t it1, int32_t kind, void* d_out,
-                int32_t es_freq = 0, double es_margin = 0.0, int32_t* d_iters = nullptr) {
+                int32_t es_freq = 0, double es_margin = 0.0, int32_t* d_iters = nullptr,
+                PredForm form = PRED_DENSE) {
   if (kind == LGBM_HIP_PREDICT_CONTRIB) {
     int32_t depth = 0, leaves = 1;
     for (int64_t t = (int64_t)it0 * m->num_tree_per_iteration;
@@ -3535,7 +3545,7 @@ int predict_run(lgbm_hip_ctx* c, const lgbm_hip_model* m, const float* d_x, int6
   const PredShape shape =
       es_freq > 0 || !c->pack.words
           ? PredShape{0, 0, 0}
-          : predict_lds_shape(rows, cols, c->pack.stride, (it1 - it0) * m->num_tree_per_iteration);
+          : predict_lds_shape(predict_call(c, m, rows, cols, it0, it1, form));
   if (shape.rb > 0) {
     PredRows R{};
     R.dense = d_x;
@@ -3637,11 +3647,11 @@ int predict_sparse(lgbm_hip_ctx* c, const lgbm_hip_model* m, const int64_t* indp
   int64_t* d_ptr = (int64_t*)(c->pm_csr + 256);
   int32_t* d_idx = (int32_t*)(c->pm_csr + 256 + pb);
   float* d_val = (float*)(c->pm_csr + 256 + pb + ib);
-  // CSR rows go straight into k_predict_lds's LDS where they fit
+  // CSR rows go straight into k_predict_lds's LDS where the call is its
   const PredShape shape =
       csc || kind == LGBM_HIP_PREDICT_CONTRIB || !c->pack.words
           ? PredShape{0, 0, 0}
-          : predict_lds_shape(num_rows, fw, c->pack.stride, (it1 - it0) * m->num_tree_per_iteration);
+          : predict_lds_shape(predict_call(c, m, num_rows, fw, it0, it1, PRED_CSR, nnz));
   const bool direct = shape.rb > 0;
   const size_t xb = direct ? 0 : (size_t)num_rows * (size_t)std::max(fw, 1) * 4;
   const size_t ob = (size_t)num_rows * (size_t)width * (kind == LGBM_HIP_PREDICT_LEAF ? 4 : 8);
@@ -3689,7 +3699,8 @@ int predict_sparse(lgbm_hip_ctx* c, const lgbm_hip_model* m, const int64_t* indp
     return set_err(c, LGBM_HIP_ERR_LENGTH_MISMATCH,
                    csc ? "csc row index out of range" : "csr column index out of range");
   if (!direct &&
-      (rc = predict_run(c, m, c->pm_x, num_rows, fw, it0, it1, kind, c->pm_out)))
+      (rc = predict_run(c, m, c->pm_x, num_rows, fw, it0, it1, kind, c->pm_out, 0, 0.0, nullptr,
+                        PRED_MADE_DENSE)))
     return rc;
   HIPCHK(c, hipMemcpy(out, c->pm_out, ob, hipMemcpyDeviceToHost));
   return LGBM_HIP_OK;

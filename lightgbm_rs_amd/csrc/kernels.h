@@ -21,6 +21,7 @@
 #pragma once
 
 #include "lgbm_device.h"
+#include "predict_shape.h"
 
 #include <hip/hip_ext.h>
 
@@ -226,7 +227,7 @@ struct DevBinFeature {
 void launch_bin_records(const void* x, int32_t f64, int32_t col_major, int64_t n, int32_t F,
                         int32_t fmt, const DevBinFeature* feats, const double* ub, int32_t ub_count,
                         const int2* cats, uint4* rec, hipStream_t s, const KernelEvents* ev);
-// k_predict_lds: the packed trees (model_pack_trees), where its rows come from, and a launch's shape.
+// k_predict_lds: the packed trees (model_pack_trees) and where its rows come from.
 struct PredPack {
   const uint2* words;
   int32_t stride, values;
@@ -241,11 +242,6 @@ struct PredRows {
   int32_t cols;
   uint32_t* err;  // bit 0: a bad indptr pair, bit 1: a bad column
 };
-struct PredShape {
-  int32_t rb, nb;  // rows and staged trees of a block
-  size_t lds;
-};
-PredShape predict_lds_shape(int64_t rows, int32_t width, int32_t tree_words, int32_t n_trees);
 int predict_lds_prepare();
 void launch_predict_lds(const PredShape& S, const PredPack& K, const int32_t* cat_bounds,
                         const uint32_t* cat_words, const PredRows& R, bool csr, int64_t rows,

@@ -678,7 +678,7 @@ bool model_pack_trees(const lgbm_hip_model& m, PredPacked* out) {
   int32_t nl = 1;
   for (const PredTree& T : m.tree_index) nl = std::max(nl, T.num_leaves);
   *out = PredPacked{};
-  if (m.any_linear || m.max_feature_idx >= 1 << 12 || 3 * (int64_t)nl - 1 > PRED_TREE_WORDS)
+  if (m.any_linear || m.max_feature_idx >= 1 << 12 || 3 * (int64_t)nl - 1 > lgbm::PRED_TREE_WORDS)
     return false;
   out->values = 2 * nl - 1;
   out->stride = 3 * nl - 1;

@@ -5,6 +5,8 @@
 #include <string>
 #include <vector>
 
+#include "predict_shape.h"
+
 // Objective ConvertOutput kinds (crates/lgbm-model/src/objective.rs:48-88).
 enum PredObjective : int32_t {
   OBJ_REGRESSION = 0,       // identity
@@ -53,7 +55,6 @@ struct PredLinLeaf {
 #define PRED_SET (1u << 29)
 #define PRED_ZERO_MISSING (1u << 30)
 #define PRED_FLIP (1u << 31)
-constexpr int32_t PRED_TREE_WORDS = 4096;  // of a tree at most, and of a staged batch
 struct PredEntry {
   float threshold;
   uint32_t word;

@@ -133,11 +133,9 @@ __device__ __forceinline__ void pred_transform(double* o, int32_t ntpi, int32_t 
   }
 }
 
-// Rows of up to this many columns are staged in LDS (256 rows x an odd stride of at
-// most 63 floats = 63 KiB): one coalesced load of the block's rows, then every tree
+// STAGE: rows of up to PRED_STAGE_COLS columns are staged in LDS (256 rows x an odd stride
+// of at most 63 floats = 63 KiB): one coalesced load of the block's rows, then every tree
 // walk reads its feature values from LDS instead of one cache line per node visit.
-constexpr int32_t PRED_STAGE_COLS = 63;
-
 template <bool STAGE>
 __global__ __launch_bounds__(256) void k_predict(PredModelDev M, const float* __restrict__ X,
                                                  int64_t rows, int32_t cols, int32_t it0,
@@ -240,10 +238,7 @@ __global__ __launch_bounds__(256) void k_predict(PredModelDev M, const float* __
 // 64 rows, 100 trees of 31 leaves 273 -> 14 us (one thread walked all trees); 200003 CSR
 // rows x 500 columns, 200 trees of 63 leaves 3.84 (with the densify) -> 1.00 ms.  Blocks
 // of half the LDS, two a CU, took 2.55 ms on the first and 2.10 on the third.
-constexpr int32_t PRED_THREADS = 1024;
 constexpr int32_t PRED_WORDS = PRED_TREE_WORDS / PRED_THREADS;  // a thread stages of a batch
-constexpr size_t PRED_LDS = 156 * 1024;
-constexpr int64_t PRED_FILL = 256;  // blocks before a block takes more rows
 
 // NODES: 0 nodes without these flags only, 1 PRED_ZERO_MISSING ones too, 2 any.  Branch-
 // free but for sets of more than a word: a wave's lanes meet all kinds at every step.
@@ -435,29 +430,6 @@ __global__ __launch_bounds__(PRED_THREADS) void k_predict_lds(
   }
   if (kind == 1 && live && g == 0)
     pred_transform(out + r * ntpi, ntpi, n_it, objective, sigmoid, average_output);
-}
-
-// Rows and trees a block takes; rb = 0 where the rows or trees do not fit.  Among the row
-// counts that leave the chip a block a CU, the one with the most walks side by side (the
-// block's LDS holds fewer trees beside more or wider rows), the larger where they tie.
-PredShape predict_lds_shape(int64_t rows, int32_t width, int32_t tree_words, int32_t n_trees) {
-  PredShape best{0, 0, 0};
-  if (n_trees < 1 || width < 1 || tree_words > PRED_TREE_WORDS) return best;
-  const size_t tree = (size_t)tree_words * 8;
-  int32_t walks = 0;
-  for (int32_t rb = PRED_THREADS; rb >= 8; rb /= 2) {
-    if (rb > 8 && rows < (int64_t)rb * PRED_FILL) continue;
-    const int32_t groups = PRED_THREADS / rb;
-    const size_t x = (size_t)rb * (size_t)(width | 1) * 4;
-    const size_t per_tree = 2 * tree + (groups > 1 ? (size_t)rb * 16 : 0);
-    if (x + per_tree > PRED_LDS) continue;
-    int64_t nb = std::min((int64_t)((PRED_LDS - x) / per_tree), (int64_t)PRED_TREE_WORDS / tree_words);
-    nb = std::min<int64_t>(std::min<int64_t>(nb, n_trees), std::max(groups, 8));
-    if (rb * (int32_t)std::min<int64_t>(nb, groups) <= walks) continue;
-    walks = rb * (int32_t)std::min<int64_t>(nb, groups);
-    best = {rb, (int32_t)nb, x + per_tree * (size_t)nb};
-  }
-  return best;
 }
 
 // Opts the kernels into their LDS; 0 = ok.

@@ -18,7 +18,7 @@ def be():
     b.close()
 
 
-def _text(rng, leaves, cols, classes, iters, cat):
+def _text(rng, leaves, cols, classes, iters, cat, infinite=False):
     out = ["tree", "version=v4", f"num_class={classes}", f"num_tree_per_iteration={classes}",
            "label_index=0", f"max_feature_idx={cols - 1}",
            "objective=" + (f"multiclass num_class:{classes}" if classes > 1 else "binary sigmoid:1"),
@@ -42,6 +42,8 @@ def _text(rng, leaves, cols, classes, iters, cat):
         thr = rng.normal(size=nl - 1)
         thr[::5] = 0.0
         thr[1::7] = np.float32(0.5)
+        if infinite:
+            thr[2::9] = np.inf
         dt = rng.choice([0, 2, 4, 6, 8, 10], nl - 1)
         is_cat = (rng.random(nl - 1) < 0.3) if cat else np.zeros(nl - 1, bool)
         dt[is_cat] = 1
@@ -103,3 +105,40 @@ def test_bits_equal_the_oracle(be, rows, repeat, cols, leaves, classes, iters, c
         part = be.predict(m, X, kind, start_iteration=1, num_iteration=1)
         ref = np.asarray(P.predict(pm, X, 1, 1, kind))
         np.testing.assert_allclose(part, ref.reshape(rows, -1), rtol=1e-14, atol=0)
+
+
+# Calls just past what the packed trees or the block's LDS take (leaves, columns, an infinite
+# threshold, wide rows beside a large tree) and one of few trees over wide rows: k_predict's.
+@pytest.mark.parametrize("rows,cols,leaves,iters,infinite", [
+    (40, 5, 1365, 2, False), (40, 5, 1366, 2, False), (30, 4096, 31, 4, False),
+    (30, 4097, 31, 4, False), (20, 5001, 15, 3, False), (90, 12, 31, 5, True),
+    (20, 4000, 900, 2, False), (300, 1000, 31, 1, False)])
+def test_either_side_of_a_limit(be, rows, cols, leaves, iters, infinite):
+    rng = np.random.default_rng(rows + cols)
+    text = _text(rng, leaves, cols, 1, iters, False, infinite)
+    m, pm = Model(text), P.parse_model(text)
+    X = _rows(rng, rows, cols)
+    sparse = X.copy()
+    sparse[rng.random(X.shape) < 0.5] = 0.0
+    r, c = np.nonzero((sparse != 0) | np.isnan(sparse))
+    ends = np.concatenate([[0], np.cumsum(np.bincount(r, minlength=rows))])
+    for kind in ("raw", "leaf"):
+        print(f"predict limit cols={cols} leaves={leaves} kind={kind}", flush=True)
+        ref = np.asarray(P.predict(pm, X, kind=kind)).reshape(rows, -1)
+        assert np.array_equal(be.predict(m, X, kind), ref)
+        ref = np.asarray(P.predict(pm, sparse, kind=kind)).reshape(rows, -1)
+        assert np.array_equal(be.predict_csr(m, ends, c, sparse[r, c], cols, kind), ref)
+
+
+@pytest.mark.parametrize("rows,extra", [(1, 1), (70, 3), (70, 972), (3000, 972), (270_000, 9)])
+def test_rows_wider_than_the_model(be, rows, extra):
+    """Columns past max_feature_idx, which no tree reads."""
+    rng = np.random.default_rng(rows + extra)
+    text = _text(rng, 31, 28, 2, 20, True)
+    m, pm = Model(text), P.parse_model(text)
+    X = _rows(rng, min(rows, 70), 28)
+    ref = np.asarray(P.predict(pm, X, kind="raw"))
+    big = np.full((rows, 28 + extra), np.nan, np.float32)
+    big[:, :28] = np.resize(X, (rows, 28))
+    print(f"predict rows={rows} extra={extra}", flush=True)
+    assert np.array_equal(be.predict(m, big, "raw"), np.resize(ref.reshape(len(X), -1), (rows, 2)))
