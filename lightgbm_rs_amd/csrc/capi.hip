@@ -146,7 +146,9 @@ struct lgbm_hip_ctx {
   PredLinLeaf* pm_linl = nullptr;
   int32_t* pm_linf = nullptr;
   double* pm_linc = nullptr;
-  PredEntry* pm_pack = nullptr;  // the packed trees of k_predict_lds (pack.words; NULL: none)
+  // the packed trees of the model of pack_uid, for k_predict_lds (pack.words; NULL: none)
+  uint64_t pack_uid = 0;
+  PredEntry* pm_pack = nullptr;
   PredPack pack{};
   bool pack_lds = false;  // the kernels were opted into their LDS
   double* pm_ncov = nullptr;  // TreeSHAP covers and expected values
@@ -3369,24 +3371,35 @@ int predict_prepare(lgbm_hip_ctx* c, const lgbm_hip_model* m, int64_t rows, int3
     if ((rc = upload_vec(c, &c->pm_ncov, m->node_cover))) return rc;
     if ((rc = upload_vec(c, &c->pm_lcov, m->leaf_cover))) return rc;
     if ((rc = upload_vec(c, &c->pm_expv, m->tree_expected))) return rc;
-    PredPacked pk;
-    c->pack = PredPack{};
-    bool packed = false;
-    try {
-      packed = model_pack_trees(*m, &pk);
-    } catch (const std::exception& e) {  // no host memory: not past the C entry
-      return set_err(c, LGBM_HIP_ERR_RUNTIME, e.what());
-    }
-    if (packed) {
-      if (!c->pack_lds && predict_lds_prepare())
-        return set_err(c, LGBM_HIP_ERR_HIP, "the prediction kernels' LDS size was refused");
-      c->pack_lds = true;
-      if ((rc = upload_vec(c, &c->pm_pack, pk.words))) return rc;
-      c->pack = PredPack{(const uint2*)c->pm_pack, pk.stride, pk.values, pk.zero, pk.cat, pk.set};
-    }
     c->pm_uid = m->uid;
   }
   return LGBM_HIP_OK;
+}
+
+// The model's packed trees, made when a call that k_predict_lds may serve first asks for
+// them.  Without them (model_pack_trees, or no memory for them here) such calls are k_predict's.
+void predict_pack(lgbm_hip_ctx* c, const lgbm_hip_model* m) {
+  if (c->pack_uid == m->uid) return;
+  c->pack_uid = m->uid;
+  c->pack = PredPack{};
+  if (c->pm_pack) (void)hipFree(c->pm_pack);
+  c->pm_pack = nullptr;
+  if (!c->pack_lds && predict_lds_prepare()) {
+    (void)hipGetLastError();
+    return;
+  }
+  c->pack_lds = true;
+  PredPacked pk;
+  if (!model_pack_trees(*m, &pk)) return;
+  const size_t bytes = pk.words.size() * sizeof(PredEntry);
+  if (hipMalloc((void**)&c->pm_pack, bytes) != hipSuccess ||
+      hipMemcpy(c->pm_pack, pk.words.data(), bytes, hipMemcpyHostToDevice) != hipSuccess) {
+    (void)hipGetLastError();  // not the call's error
+    if (c->pm_pack) (void)hipFree(c->pm_pack);
+    c->pm_pack = nullptr;
+    return;
+  }
+  c->pack = PredPack{(const uint2*)c->pm_pack, pk.stride, pk.values, pk.zero, pk.cat, pk.set};
 }
 
 // Feature contributions of iterations [it0, it1) by leaf paths (k_shap_items): the trees
@@ -3542,6 +3555,7 @@ int predict_run(lgbm_hip_ctx* c, const lgbm_hip_model* m, const float* d_x, int6
     return LGBM_HIP_OK;
   }
   KernelEvents ke;
+  if (es_freq <= 0) predict_pack(c, m);
   const PredShape shape =
       es_freq > 0 || !c->pack.words
           ? PredShape{0, 0, 0}
@@ -3648,6 +3662,7 @@ int predict_sparse(lgbm_hip_ctx* c, const lgbm_hip_model* m, const int64_t* indp
   int32_t* d_idx = (int32_t*)(c->pm_csr + 256 + pb);
   float* d_val = (float*)(c->pm_csr + 256 + pb + ib);
   // CSR rows go straight into k_predict_lds's LDS where the call is its
+  if (kind != LGBM_HIP_PREDICT_CONTRIB) predict_pack(c, m);
   const PredShape shape =
       csc || kind == LGBM_HIP_PREDICT_CONTRIB || !c->pack.words
           ? PredShape{0, 0, 0}

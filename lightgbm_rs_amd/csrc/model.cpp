@@ -674,62 +674,96 @@ void model_shap_paths(const lgbm_hip_model& m, ShapPaths* out) {
   }
 }
 
-bool model_pack_trees(const lgbm_hip_model& m, PredPacked* out) {
-  int32_t nl = 1;
-  for (const PredTree& T : m.tree_index) nl = std::max(nl, T.num_leaves);
-  *out = PredPacked{};
-  if (m.any_linear || m.max_feature_idx >= 1 << 12 || 3 * (int64_t)nl - 1 > lgbm::PRED_TREE_WORDS)
+namespace {
+
+// The largest float below f, which is not NaN and not -inf.
+float float_below(float f) {
+  uint32_t b;
+  std::memcpy(&b, &f, 4);
+  b = (b << 1) == 0u ? 0x80000001u : (b >> 31) ? b + 1 : b - 1;
+  std::memcpy(&f, &b, 4);
+  return f;
+}
+
+bool pack_trees(const lgbm_hip_model& m, PredPacked* out) {
+  int64_t nl = 1, tight = 0;
+  for (const PredTree& T : m.tree_index) {
+    nl = std::max<int64_t>(nl, T.num_leaves);
+    tight += 3 * (int64_t)T.num_leaves - 1;
+  }
+  if (m.any_linear || m.max_feature_idx >= 1 << 12 || 3 * nl - 1 > lgbm::PRED_TREE_WORDS)
     return false;
-  out->values = 2 * nl - 1;
-  out->stride = 3 * nl - 1;
-  // bounded: a model of a few very large trees among many small ones is not worth it
-  if ((int64_t)m.tree_index.size() * out->stride > (int64_t)1 << 26) return false;
-  out->words.assign(m.tree_index.size() * (size_t)out->stride, PredEntry{0.0f, 0u});
+  out->values = (int32_t)(2 * nl - 1);
+  out->stride = (int32_t)(3 * nl - 1);
+  // every tree takes the largest one's words: not where that is mostly padding, past the 64 MiB
+  // that any model may take
+  const int64_t total = (int64_t)m.tree_index.size() * out->stride;
+  if (total > (int64_t)1 << 26 || total > std::max((int64_t)1 << 23, 8 * tight)) return false;
+  out->words.assign((size_t)total, PredEntry{0.0f, 0u});
+  struct At {
+    int32_t node, entry;
+  };
+  std::vector<At> at;
   for (size_t t = 0; t < m.tree_index.size(); ++t) {
     const PredTree& T = m.tree_index[t];
     PredEntry* w = out->words.data() + t * (size_t)out->stride;
     std::memcpy((void*)(w + out->values), m.leaf_values.data() + T.leaf0, (size_t)T.num_leaves * 8);
     if (T.num_leaves <= 1) continue;  // entry 0 is leaf 0
-    std::vector<int32_t> at{0};  // entry -> node (or ~leaf), in entry order
-    for (size_t e = 0; e < at.size(); ++e) {
-      if (at[e] < 0) {
-        const uint32_t leaf = (uint32_t)~at[e];
-        std::memcpy(&w[e].threshold, &leaf, 4);
-        continue;
-      }
-      const PredNode& n = m.nodes[(size_t)T.node0 + (size_t)at[e]];
-      w[e].word = (uint32_t)at.size() | (uint32_t)n.feature << 16;
-      bool right_first = false;
+    // the nodes in entry order, each placing its children (no branch on what a child is or
+    // which comes first: both are as good as random)
+    at.resize((size_t)T.num_leaves + 1);
+    at[0] = At{0, 0};
+    for (int32_t i = 0, found = 1, next = 1; i < found; ++i, next += 2) {
+      const PredNode& n = m.nodes[(size_t)T.node0 + (size_t)at[i].node];
+      PredEntry& E = w[at[i].entry];
+      E.word = (uint32_t)next | (uint32_t)n.feature << 16;
+      int32_t child[2] = {n.left, n.right};
       if (n.dtype & 1) {
         const size_t set = (size_t)T.cat0 + (size_t)n.threshold;
         const int32_t lo = m.cat_bounds[set], words = m.cat_bounds[set + 1] - lo;
         const uint32_t bits = words > 1 ? (uint32_t)set : words ? m.cat_words[(size_t)lo] : 0u;
-        std::memcpy(&w[e].threshold, &bits, 4);
-        w[e].word |= PRED_CATEGORICAL | (words > 1 ? PRED_SET : 0u);
+        std::memcpy(&E.threshold, &bits, 4);
+        E.word |= PRED_CATEGORICAL | (words > 1 ? PRED_SET : 0u);
         out->cat = true;
         out->set = out->set || words > 1;
       } else {
         // the largest float not above the threshold: f32 values compare with it alike
         float f = (float)n.threshold;
-        if ((double)f > n.threshold) f = std::nextafterf(f, -INFINITY);
+        if (!(std::fabs(n.threshold) < INFINITY)) return false;
+        f = (double)f > n.threshold ? float_below(f) : f;
         if (!(std::fabs(f) < INFINITY)) return false;
         const int32_t missing = (n.dtype >> 2) & 3;
         const bool left = missing == 1 || missing == 2 ? (n.dtype & 2) != 0 : 0.0 <= n.threshold;
         if (missing == 1) {
-          w[e].word |= PRED_ZERO_MISSING;
+          E.word |= PRED_ZERO_MISSING;
           out->zero = true;
         }
-        if (!left) {
-          // v <= f, which a NaN fails: -v > the float below -f
-          right_first = true;
-          f = std::nextafterf(-f, -INFINITY);
-          w[e].word |= PRED_FLIP;
-        }
-        w[e].threshold = f;
+        // where a NaN goes right: v <= f, which it fails, is -v > the float below -f
+        const float below = float_below(-f);
+        E.threshold = left ? f : below;
+        E.word |= left ? 0u : PRED_FLIP;
+        child[0] = left ? n.left : n.right;
+        child[1] = left ? n.right : n.left;
       }
-      at.push_back(right_first ? n.right : n.left);
-      at.push_back(right_first ? n.left : n.right);
+      for (int k = 0; k < 2; ++k) {
+        const int32_t c = child[k], leaf = ~c;
+        std::memcpy(&w[next + k].threshold, &leaf, 4);  // a leaf's entry, or rewritten
+        at[found] = At{c, next + k};
+        found += c >= 0 ? 1 : 0;
+      }
     }
   }
   return true;
+}
+
+}  // namespace
+
+bool model_pack_trees(const lgbm_hip_model& m, PredPacked* out) noexcept {
+  *out = PredPacked{};
+  try {
+    if (pack_trees(m, out)) return true;
+  } catch (...) {  // no memory
+  }
+  *out = PredPacked{};
+  return false;
 }

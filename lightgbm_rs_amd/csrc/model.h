@@ -142,12 +142,13 @@ struct ShapPaths {
   std::vector<int32_t> feats;
 };
 void model_shap_paths(const lgbm_hip_model& m, ShapPaths* out);
-// Every tree's entries and leaf values, `stride` words a tree; false where a tree or
-// feature is too large for the form, a leaf is linear or a threshold infinite or NaN.
+// Every tree's entries and leaf values, `stride` words a tree.  They are only a faster form:
+// false (and nothing made) where a tree or feature is too large for it, a leaf is linear, a
+// threshold infinite or NaN, or memory is short, and k_predict walks the nodes instead.
 struct PredPacked {
   std::vector<PredEntry> words;
   int32_t stride = 0, values = 0;
   // whether any node has PRED_ZERO_MISSING, PRED_CATEGORICAL, PRED_SET
   bool zero = false, cat = false, set = false;
 };
-bool model_pack_trees(const lgbm_hip_model& m, PredPacked* out);
+bool model_pack_trees(const lgbm_hip_model& m, PredPacked* out) noexcept;
