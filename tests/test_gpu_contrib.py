@@ -4,10 +4,10 @@ the real LightGBM binary's captures and the oracle.
 Bars: f64 bits equal to the real binary's `pred_contrib` captures
 (predict_modes/{numeric,categorical,multiclass}/contrib.txt); bits equal to the
 oracle on seeded rows with NaNs for the committed model texts (numeric, categorical,
-multiclass, missing-value handling) and for iteration slices; on 1M rows, which run
-as two workspace chunks, the reference's invariant (per class the contributions and
-the base sum to the raw score of the device predictor, within 1e-12) and the oracle's
-bits on rows around the chunk boundary."""
+multiclass, missing-value handling) and for iteration slices; on 1M rows the reference's
+invariant (per class the contributions and the base sum to the raw score of the device
+predictor, within 1e-12) and the oracle's bits at both ends and between.  Calls whose
+values or paths are cut into chunks: test_gpu_contrib_paths.py."""
 import os
 
 import numpy as np
@@ -58,7 +58,7 @@ def test_device_contrib_vs_oracle(be, name):
         assert np.array_equal(bits(got), bits(ref))
 
 
-def test_device_contrib_large_two_chunks(be):
+def test_device_contrib_large(be):
     print("contrib 1M rows", flush=True)
     text, X0, _ = PM.contrib("numeric")
     m, pm = Model(text), P.parse_model(text)
@@ -71,12 +71,7 @@ def test_device_contrib_large_two_chunks(be):
     raw = be.predict(m, X, "raw")
     np.testing.assert_allclose(got.reshape(len(X), -1, nf + 1).sum(axis=2), raw, rtol=0,
                                atol=1e-12)
-    # a workspace chunk holds (256 MiB / bytes per row) rows rounded down to 256
-    depth = max(P._max_depth(t) for t in pm["trees"])
-    per_row = (depth + 1) * (depth + 2) // 2 * 28 + (depth + 1) * 24
-    chunk = (256 << 20) // per_row // 256 * 256
-    assert chunk < len(X)
-    for r0 in (0, chunk - 150, len(X) - 300):
+    for r0 in (0, 500_000, len(X) - 300):
         sl = slice(r0, r0 + 300)
         assert np.array_equal(bits(got[sl]), bits(P.predict_contrib(pm, X[sl])))
 

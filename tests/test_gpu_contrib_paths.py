@@ -3,7 +3,8 @@ them and the one-thread-per-row kernel.  Bar: f64 bits equal to the oracle's rec
 
 Trees are random with repeated features on their paths, from balanced ones to a chain of
 SHAP_MAX_DEPTH = 31 levels (the deepest the leaf paths take) and one level more; rows from
-fewer than any leaf's outcomes (items are rows) to more (items are outcomes)."""
+fewer than any leaf's outcomes (items are rows) to more (items are outcomes), and so many
+that the values are cut into runs of trees, chunks of rows, or k_contrib's chunks."""
 import numpy as np
 import pytest
 
@@ -79,3 +80,87 @@ def test_consecutive_leaves_meet_the_same_features(be, cols):
     X = rng.normal(size=(70, cols)).astype(np.float32)
     got, ref = be.predict(m, X, "contrib"), P.predict_contrib(P.parse_model(m.to_text()), X)
     assert np.array_equal(got.view(np.uint64), np.ascontiguousarray(ref).view(np.uint64))
+
+
+VALUES = 1 << 25  # of a launch of k_shap_items
+
+
+def _comb(rng, leaves, cols, spine):
+    """A chain of `spine` levels above a random subtree of the other leaves."""
+    t, sub = _tree(rng, leaves, cols, True), _tree(rng, leaves - spine, cols, False)
+    for side in ("left_child", "right_child"):
+        t[side] = np.concatenate([t[side][:spine],
+                                  [k + spine if k >= 0 else ~(~k + spine) for k in sub[side]]])
+    return t
+
+
+def _paths(t):
+    """(depth, length of the unique path) of every leaf."""
+    out, todo = [], [(0, ())]
+    while todo:
+        node, feats = todo.pop()
+        if node < 0:
+            out.append((len(feats), len(set(feats))))
+            continue
+        feats += (int(t["split_feature"][node]),)
+        todo += [(int(t["left_child"][node]), feats), (int(t["right_child"][node]), feats)]
+    return out
+
+
+def _values(t, rows):
+    return sum(min(rows, 2 ** d) * m for d, m in _paths(t))
+
+
+def _check_slices(be, m, X, starts):
+    got = be.predict(m, X, "contrib")
+    pm = P.parse_model(m.to_text())
+    for r0 in starts:
+        sl = slice(r0, r0 + 6)
+        ref = np.ascontiguousarray(P.predict_contrib(pm, X[sl]))
+        assert np.array_equal(got[sl].view(np.uint64), ref.view(np.uint64)), r0
+
+
+def test_trees_in_two_runs(be):
+    """The second run goes on from the first one's sums, within an iteration of three classes."""
+    rng, rows, cols = np.random.default_rng(1), 20_000, 12
+    m = Model.create(num_class=3, max_feature_idx=cols - 1)
+    trees = [_tree(rng, 32, cols, True) for _ in range(9)]
+    for t in trees:
+        m.add_tree(t)
+    sizes = [_values(t, rows) for t in trees]
+    first = next(i for i in range(9) if sum(sizes[:i + 1]) > VALUES)
+    assert max(sizes) <= VALUES and 0 < first < 9 and first % 3
+    print(f"contrib runs of {first} and {9 - first} trees", flush=True)
+    X = rng.normal(size=(rows, cols)).astype(np.float32)
+    _check_slices(be, m, X, (0, 9_000, rows - 6))
+
+
+def test_rows_in_chunks(be):
+    """A tree whose values of all rows are too many: chunks of rows, the last one shorter
+    than the items that the plan has for a chunk."""
+    rng, rows, cols = np.random.default_rng(2), 40_001, 24
+    m = Model.create(num_class=1, max_feature_idx=cols - 1)
+    trees = [_comb(rng, 200, cols, 13), _tree(rng, 20, cols, False)]
+    for t in trees:
+        m.add_tree(t)
+    assert max(d for d, _ in _paths(trees[0])) <= 31
+    chunk = rows
+    while max(_values(t, chunk) for t in trees) > VALUES:
+        chunk = (chunk + 1) // 2
+    assert 0 < rows % chunk and rows > 2 * chunk and any(2 ** d > chunk for d, _ in _paths(trees[0]))
+    print(f"contrib chunks of {chunk} of {rows} rows", flush=True)
+    X = rng.normal(size=(rows, cols)).astype(np.float32)
+    _check_slices(be, m, X, (0, chunk - 3, 2 * chunk - 3, rows - 6))
+
+
+def test_k_contrib_in_two_chunks(be):
+    """A tree deeper than the leaf paths take, over more rows than its path workspace holds."""
+    rng, cols, depth = np.random.default_rng(3), 12, 32
+    per_row = (depth + 1) * (depth + 2) // 2 * 28 + (depth + 1) * 24
+    chunk = (256 << 20) // per_row // 256 * 256
+    m = Model.create(num_class=1, max_feature_idx=cols - 1)
+    for leaves in (depth + 1, 9):
+        m.add_tree(_tree(rng, leaves, cols, True))
+    print(f"contrib deep chunks of {chunk} rows", flush=True)
+    X = rng.normal(size=(chunk + 500, cols)).astype(np.float32)
+    _check_slices(be, m, X, (0, chunk - 3, chunk + 494))
