@@ -77,10 +77,11 @@ struct ShapPlan {
   uint32_t off, items;
 };
 #define SHAP_BY_ROW 0x80000000u
-// The deepest and widest trees taken this way (one wave's LDS holds a path's weights, a
-// block's the leaves of its rows).
+// The deepest and widest trees taken this way: a wave's LDS holds a path's weights, and a
+// block's holds 8 rows' sums and leaves at least (shap_rows_per_block), so that 1 feature
+// leaves room for 908 leaves, 28 for 884, 100 for 820 and 500 for 464.
 constexpr int32_t SHAP_MAX_DEPTH = 31;
-constexpr int32_t SHAP_MAX_LEAVES = 1024;
+constexpr int32_t SHAP_MAX_LEAVES = 908;
 
 struct HostTree {
   int32_t num_leaves = 0, num_cat = 0;

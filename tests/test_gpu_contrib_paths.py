@@ -2,9 +2,10 @@
 them and the one-thread-per-row kernel.  Bar: f64 bits equal to the oracle's recursion.
 
 Trees are random with repeated features on their paths, from balanced ones to a chain of
-SHAP_MAX_DEPTH = 31 levels (the deepest the leaf paths take) and one level more; rows from
-fewer than any leaf's outcomes (items are rows) to more (items are outcomes), and so many
-that the values are cut into runs of trees, chunks of rows, or k_contrib's chunks."""
+SHAP_MAX_DEPTH = 31 levels (the deepest the leaf paths take) and one level more, and of up
+to SHAP_MAX_LEAVES = 908 leaves and one more; rows from fewer than any leaf's outcomes
+(items are rows) to more (items are outcomes), and so many that the values are cut into
+runs of trees, chunks of rows, or k_contrib's chunks."""
 import numpy as np
 import pytest
 
@@ -78,6 +79,18 @@ def test_consecutive_leaves_meet_the_same_features(be, cols):
         m.add_tree(t)
     print(f"contrib rotating features cols={cols}", flush=True)
     X = rng.normal(size=(70, cols)).astype(np.float32)
+    got, ref = be.predict(m, X, "contrib"), P.predict_contrib(P.parse_model(m.to_text()), X)
+    assert np.array_equal(got.view(np.uint64), np.ascontiguousarray(ref).view(np.uint64))
+
+
+# the widest trees of one feature and of 28 whose rows fit k_shap_rows's LDS, and one leaf more
+@pytest.mark.parametrize("leaves,cols", [(908, 1), (909, 1), (884, 28), (885, 28)])
+def test_either_side_of_the_leaf_limit(be, leaves, cols):
+    rng = np.random.default_rng(leaves)
+    m = Model.create(num_class=1, max_feature_idx=cols - 1)
+    m.add_tree(_tree(rng, leaves, cols, False))
+    print(f"contrib leaves={leaves} cols={cols}", flush=True)
+    X = rng.normal(size=(3, cols)).astype(np.float32)
     got, ref = be.predict(m, X, "contrib"), P.predict_contrib(P.parse_model(m.to_text()), X)
     assert np.array_equal(got.view(np.uint64), np.ascontiguousarray(ref).view(np.uint64))
 
