@@ -51,12 +51,11 @@
 // of the adds out measured no gain), so fewer, longer chunks are faster: 1M x 2000, f32, ten
 // trees of 127 leaves, 1024 / 512 / 256 blocks 76.2 / 74.7 / 73.3 ms; 2M x 100 x 10 classes
 // 48.1 / 47.3 / 47.6; 2M x 700 quantized, ten trees of 255 leaves, 512 / 256 / 128 blocks
-// 94.1 / 93.3 / 98.0.  Past WIDE_GRID_GROUPS groups, whole chunks of all groups leave up to a
-// third of the CUs without a block, and the larger grids stay.
+// 94.1 / 93.3 / 98.0.  That holds whatever 256 leaves over when divided among the groups:
+// 200k rows, f32, three trees of 63 leaves, 1024 -> 256 blocks, 44 groups 7.72 -> 7.24 ms, 60
+// 9.34 -> 8.68, 65 9.98 -> 9.58, 85 11.81 -> 11.26, 125 15.62 -> 14.45 (90 % zeros: 1 to 5 %
+// less); 1100 columns of 1000 bins 24.5 -> 23.5 ms, quantized 22.0 -> 21.3.
 #define WIDE_GRID 256
-#define WIDE_GRID_GROUPS 64
-#define WIDE_GRID_MANY_Q 512
-#define WIDE_GRID_MANY_F 1024
 #ifndef WIDE_MIN_ROWS
 #define WIDE_MIN_ROWS 4096              // rows per chunk (at least): a flush costs a group
 #endif

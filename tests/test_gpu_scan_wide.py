@@ -1,6 +1,6 @@
 """Child scans of the wide layout (k_pair_scan_wide): features of 1 to 256 bins side by side,
 an odd number of them, most frequent bins at either end and between, children too small to
-split, against the oracle.  Bar: quantized trees bit-exact; f32 ones equal in structure,
+split, more than 64 feature groups of histograms, against the oracle.  Bar: quantized trees bit-exact; f32 ones equal in structure,
 leaf values within 1e-9 (one rounding of a fixed-point sum a cell against the f64 fold)."""
 import numpy as np
 import pytest
@@ -53,7 +53,7 @@ def _check(n, F, leaves, quant, cfg, max_depth=-1, contri=None):
 
 @pytest.mark.parametrize("quant", [True, False])
 @pytest.mark.parametrize("n,F,leaves,min_data", [(300, 125, 15, 5), (5000, 131, 63, 1),
-                                                 (20_000, 200, 40, 50)])
+                                                 (20_000, 200, 40, 50), (3000, 2100, 15, 5)])
 def test_trees_match_the_oracle(n, F, leaves, min_data, quant):
     print(f"wide scans n={n} F={F} quant={quant}", flush=True)
     _check(n, F, leaves, quant, GainConfig.make(min_data_in_leaf=min_data))
