@@ -179,9 +179,12 @@ __host__ __device__ inline int64_t part_span_blocks(int64_t t0, int64_t n, int64
 // Record layouts, f32 gradients: the rows of the smaller child up to which k_pair_scan adds
 // its histogram itself, a feature a block, instead of k_hist_f32, whose blocks clear and
 // store every cell of their features whatever the rows.  Trainings of 1e5 to 3e6 rows
-// measured alike at 512 to 4096; data of at most HIST_FP_ALL_DIRECT rows leaves every child
-// to the scan, and its rounds have no k_hist_f32 launch (5003 rows x 13 features, 20 trees
-// of 31 leaves: 11.5 -> 10.7 ms).
+// measured alike at 512 to 4096.  Data of at most HIST_FP_ALL_DIRECT rows leaves every child
+// to the scan, and its rounds have no k_hist_f32 launch: ten trees of 31 leaves at 1000, 3000,
+// 5003 and 8000 rows, ms with the launch and without, 13 columns 5.54/5.17, 5.68/5.28,
+// 5.79/5.27, 5.16/4.77; 30 columns 5.41/4.87, 5.63/5.06, 5.53/4.99, 5.28/4.75; 39 columns of
+// 63 bins 4.67/4.32, 4.93/4.49, 4.94/4.41, 4.73/4.12.  The line is below the crossing: without
+// the launch 12000 to 30000 rows took 0.85 to 0.97 times theirs at these columns.
 __host__ __device__ inline int64_t hist_fp_direct(int64_t N) {
   return N <= HIST_FP_ALL_DIRECT ? N : HIST_FP_DIRECT;
 }
