@@ -696,11 +696,17 @@ __global__ __launch_bounds__(256) void k_hist_reduce64(DevLearner L) {
 // the job's accumulator (L.hist_acc64, read and cleared by k_pair_scan), whose reader
 // would else sum hundreds of slots one by one.
 //
-// The features of a group are walked with their word, shift and first cell known at
-// compile time or in scalar registers: two atomics and four VALU instructions a (row,
-// feature).  Read from LDS tables per feature, with the word picked by masking them all,
-// it was bound by VALU: 1M rows x 28 features of 255 bins, all builds of a tree of 63
-// leaves, 613 us.
+// The features of a group are walked with their word and shift known at compile time and
+// their first cell in a scalar register, or, where the record's features are more than the
+// scalar registers hold (28 columns spill 66 of them, 60 columns 307, 124 columns 578), in a
+// lane of a vector register: two atomics and four VALU instructions a (row, feature), and
+// there a lane read.  Read from LDS tables per feature, with the word picked by masking them
+// all, it was bound by VALU: 1M rows x 28 features of 255 bins, all builds of a tree of 63
+// leaves, 613 us.  Five trees of 63 leaves from that form to this one with the accumulators
+// and the children that the scan builds, 200k and 1M rows, ms: 12 columns 4.54 -> 3.23, 6.79
+// -> 4.12; 28 columns 5.35 -> 3.60, 8.02 -> 5.08; 60 columns 5.20 -> 4.64, 7.61 -> 6.33; 92
+// columns 5.36 -> 4.75, 8.79 -> 7.00; 124 columns 5.41 -> 4.83, 9.38 -> 7.53; 39 columns of 63
+// bins 8.11 -> 3.54, 9.74 -> 4.73.
 template <int FMT>
 __global__ __launch_bounds__(HIST_THREADS, 2) void k_hist_f32(DevLearner L) {
   constexpr int U = rec_words(FMT), BPW = rec_bpw(FMT), BB = rec_bits(FMT), NS = rec_slots(FMT);
