@@ -36,8 +36,8 @@ void launch_shap_paths(const PredNode* nodes, const PredTree* trees, const doubl
                        const int32_t* cat_bounds, const uint32_t* cat_words,
                        const double* node_cover, const double* leaf_cover, const double* expected,
                        const ShapLeaf* leaves, const ShapStep* steps, const int32_t* feats,
-                       const ShapPlan* plan, int64_t max_items, const float* X, int64_t rows,
-                       int32_t cols, int32_t nf, int32_t max_leaves, int32_t t0, int32_t t1,
+                       const ShapPlan* plan, int32_t base, int64_t max_items, const float* X,
+                       int64_t rows, int32_t cols, int32_t nf, int32_t max_leaves, int32_t t0, int32_t t1,
                        int32_t leaf0, int32_t leaf1, int32_t ntpi, int first, double* tab,
                        double* out, hipStream_t s);
 void launch_csr_dense(const int64_t* indptr, const int32_t* indices, const float* values,
@@ -158,9 +158,11 @@ struct lgbm_hip_ctx {
   size_t pm_csr_cap = 0;
   char* pm_shap = nullptr;  // TreeSHAP path workspace
   size_t pm_shap_cap = 0;
-  // the leaf paths of the model of pm_paths_uid (made when contributions are first asked
-  // of it), their depths and lengths on the host, and the last call's plan
+  // the leaf paths of trees [pm_paths_t0, pm_paths_t1) of the model of pm_paths_uid (made when
+  // contributions of a range beyond them are asked for), their depths and lengths on the
+  // host, and the last call's plan
   uint64_t pm_paths_uid = 0;
+  int32_t pm_paths_t0 = 0, pm_paths_t1 = 0;
   ShapLeaf* pm_sleaf = nullptr;
   ShapStep* pm_sstep = nullptr;
   int32_t* pm_sfeat = nullptr;
@@ -3409,19 +3411,25 @@ int contrib_paths(lgbm_hip_ctx* c, const lgbm_hip_model* m, const float* d_x, in
   int rc = 0;
   const int32_t ntpi = m->num_tree_per_iteration, nf = m->max_feature_idx + 1;
   const int32_t nt0 = it0 * ntpi, nt1 = it1 * ntpi;
-  const size_t nleaf = m->leaf_values.size();
-  if (c->pm_paths_uid != m->uid) {
+  if (c->pm_paths_uid != m->uid || nt0 < c->pm_paths_t0 || nt1 > c->pm_paths_t1) {
     c->pm_paths_uid = 0;
     ShapPaths p;
-    model_shap_paths(*m, &p);
+    model_shap_paths(*m, nt0, nt1, &p);
     if ((rc = upload_vec(c, &c->pm_sleaf, p.leaves))) return rc;
     if ((rc = upload_vec(c, &c->pm_sstep, p.steps))) return rc;
     if ((rc = upload_vec(c, &c->pm_sfeat, p.feats))) return rc;
-    if ((rc = dalloc(c, &c->pm_splan, nleaf))) return rc;
-    c->shap_dm.resize(nleaf);
-    for (size_t l = 0; l < nleaf; ++l) c->shap_dm[l] = p.leaves[l].dm;
+    if ((rc = dalloc(c, &c->pm_splan, p.leaves.size()))) return rc;
+    c->shap_dm.resize(p.leaves.size());
+    for (size_t l = 0; l < p.leaves.size(); ++l) c->shap_dm[l] = p.leaves[l].dm;
     c->pm_paths_uid = m->uid;
+    c->pm_paths_t0 = nt0;
+    c->pm_paths_t1 = nt1;
   }
+  // leaves count from the paths' first one; the plan has those of the call's trees
+  const int32_t base = m->tree_index[(size_t)c->pm_paths_t0].leaf0;
+  const size_t leaf0 = (size_t)(m->tree_index[(size_t)nt0].leaf0 - base);
+  const PredTree& end = m->tree_index[(size_t)nt1 - 1];
+  const size_t nleaf = (size_t)(end.leaf0 + end.num_leaves - base) - leaf0;
   // values of a tree whose launch covers R rows: a leaf's items are the outcomes of its
   // ancestors, or the rows where they are no more
   auto items_of = [&](size_t leaf, int64_t R) {
@@ -3432,7 +3440,7 @@ int contrib_paths(lgbm_hip_ctx* c, const lgbm_hip_model* m, const float* d_x, in
     const PredTree& T = m->tree_index[(size_t)t];
     int64_t v = 0;
     for (int32_t l = 0; l < T.num_leaves; ++l)
-      v += items_of((size_t)T.leaf0 + l, R) * (c->shap_dm[(size_t)T.leaf0 + l] >> 16);
+      v += items_of((size_t)(T.leaf0 - base) + l, R) * (c->shap_dm[(size_t)(T.leaf0 - base) + l] >> 16);
     return v;
   };
   const int64_t most = ((int64_t)256 << 20) / 8;
@@ -3454,10 +3462,10 @@ int contrib_paths(lgbm_hip_ctx* c, const lgbm_hip_model* m, const float* d_x, in
       used = 0;
     }
     for (int32_t l = 0; l < T.num_leaves; ++l) {
-      const size_t leaf = (size_t)T.leaf0 + l;
+      const size_t leaf = (size_t)(T.leaf0 - base) + l;
       const int64_t items = items_of(leaf, chunk);
       const bool by_row = items > 0 && items < ((int64_t)1 << (c->shap_dm[leaf] & 0xffff));
-      plan[leaf] = ShapPlan{(uint32_t)used, (uint32_t)items | (by_row ? SHAP_BY_ROW : 0u)};
+      plan[leaf - leaf0] = ShapPlan{(uint32_t)used, (uint32_t)items | (by_row ? SHAP_BY_ROW : 0u)};
       used += items * (c->shap_dm[leaf] >> 16);
       runs.back().items = std::max(runs.back().items, items);
     }
@@ -3470,7 +3478,7 @@ int contrib_paths(lgbm_hip_ctx* c, const lgbm_hip_model* m, const float* d_x, in
     if ((rc = dalloc(c, &c->pm_shap, need))) return rc;
     c->pm_shap_cap = need;
   }
-  HIPCHK(c, hipMemcpyAsync(c->pm_splan, plan.data(), nleaf * sizeof(ShapPlan),
+  HIPCHK(c, hipMemcpyAsync(c->pm_splan + leaf0, plan.data(), nleaf * sizeof(ShapPlan),
                            hipMemcpyHostToDevice, c->stream));
   const int64_t width = (int64_t)ntpi * (nf + 1);
   for (int64_t r0 = 0; r0 < rows; r0 += chunk)
@@ -3479,7 +3487,7 @@ int contrib_paths(lgbm_hip_ctx* c, const lgbm_hip_model* m, const float* d_x, in
       const PredTree& last = m->tree_index[(size_t)R.t1 - 1];
       launch_shap_paths(c->pm_nodes, c->pm_trees, c->pm_leaves, c->pm_catb, c->pm_catw,
                         c->pm_ncov, c->pm_lcov, c->pm_expv, c->pm_sleaf, c->pm_sstep,
-                        c->pm_sfeat, c->pm_splan, R.items, d_x + r0 * cols,
+                        c->pm_sfeat, c->pm_splan, base, R.items, d_x + r0 * cols,
                         std::min(chunk, rows - r0), cols, nf, max_leaves, R.t0, R.t1,
                         m->tree_index[(size_t)R.t0].leaf0, last.leaf0 + last.num_leaves, ntpi,
                         i == 0, (double*)c->pm_shap, d_out + r0 * width, c->stream);
@@ -3520,14 +3528,16 @@ int predict_run(lgbm_hip_ctx* c, const lgbm_hip_model* m, const float* d_x, int6
                 PredForm form = PRED_DENSE) {
   if (kind == LGBM_HIP_PREDICT_CONTRIB) {
     int32_t depth = 0, leaves = 1;
+    int64_t total = 0;
     for (int64_t t = (int64_t)it0 * m->num_tree_per_iteration;
          t < (int64_t)it1 * m->num_tree_per_iteration; ++t) {
       depth = std::max(depth, m->tree_depth[t]);
       leaves = std::max(leaves, m->tree_index[t].num_leaves);
+      total += m->tree_index[t].num_leaves;
     }
     if (it0 < it1 && depth <= SHAP_MAX_DEPTH && leaves <= SHAP_MAX_LEAVES &&
         shap_rows_per_block(m->max_feature_idx + 1, leaves) > 0 &&
-        m->leaf_values.size() < (size_t)1 << 22)  // feature offsets fit 27 bits
+        total < (int64_t)1 << 22)  // feature offsets fit 27 bits
       try {
         return contrib_paths(c, m, d_x, rows, cols, it0, it1, leaves, (double*)d_out);
       } catch (const std::exception& e) {

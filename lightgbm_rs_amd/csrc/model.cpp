@@ -618,11 +618,12 @@ bool parse_model_text(const char* text, size_t len, lgbm_hip_model* m, std::stri
   return true;
 }
 
-void model_shap_paths(const lgbm_hip_model& m, ShapPaths* out) {
-  out->leaves.assign(m.leaf_values.size(), ShapLeaf{});
+void model_shap_paths(const lgbm_hip_model& m, int32_t t0, int32_t t1, ShapPaths* out) {
+  const PredTree &first = m.tree_index[(size_t)t0], &last = m.tree_index[(size_t)t1 - 1];
+  out->leaves.assign((size_t)(last.leaf0 + last.num_leaves - first.leaf0), ShapLeaf{});
   out->steps.clear();
   out->feats.clear();
-  for (size_t t = 0; t < m.tree_index.size(); ++t) {
+  for (size_t t = (size_t)t0; t < (size_t)t1; ++t) {
     const PredTree& T = m.tree_index[t];
     if (T.num_leaves <= 1 || T.num_leaves > SHAP_MAX_LEAVES || m.tree_depth[t] > SHAP_MAX_DEPTH)
       continue;
@@ -656,7 +657,7 @@ void model_shap_paths(const lgbm_hip_model& m, ShapPaths* out) {
         todo.push_back({n.left, d.depth + 1, {at, count(n.right) << 1}});
         continue;
       }
-      ShapLeaf& L = out->leaves[(size_t)T.leaf0 + (size_t)~d.node];
+      ShapLeaf& L = out->leaves[(size_t)(T.leaf0 - first.leaf0) + (size_t)~d.node];
       L.path0 = (int32_t)out->steps.size();
       L.feat0 = (int32_t)out->feats.size();
       L.tree = (int32_t)t;

@@ -135,14 +135,14 @@ std::string model_to_text(const lgbm_hip_model& m);
 bool model_add_tree(lgbm_hip_model* m, HostTree&& t, std::string* err);
 // Parses the objective line into m->objective / m->sigmoid.
 bool model_set_objective(lgbm_hip_model* m, const std::string& line, std::string* err);
-// Every leaf's path, by the index of its value; leaves of a tree that is deeper or wider
-// than the limits get none.
+// The path of every leaf of trees [t0, t1), from the first one's leaf 0 on; leaves of a tree
+// that is deeper or wider than the limits get none.
 struct ShapPaths {
   std::vector<ShapLeaf> leaves;
   std::vector<ShapStep> steps;
   std::vector<int32_t> feats;
 };
-void model_shap_paths(const lgbm_hip_model& m, ShapPaths* out);
+void model_shap_paths(const lgbm_hip_model& m, int32_t t0, int32_t t1, ShapPaths* out);
 // Every tree's entries and leaf values, `stride` words a tree.  They are only a faster form:
 // false (and nothing made) where a tree or feature is too large for it, a leaf is linear, a
 // threshold infinite or NaN, or memory is short, and k_predict walks the nodes instead.

@@ -177,3 +177,18 @@ def test_k_contrib_in_two_chunks(be):
     print(f"contrib deep chunks of {chunk} rows", flush=True)
     X = rng.normal(size=(chunk + 500, cols)).astype(np.float32)
     _check_slices(be, m, X, (0, chunk - 3, chunk + 494))
+
+
+def test_ranges_of_one_model(be):
+    """Calls of ranges within, across and beyond the trees whose paths are there already."""
+    rng, cols, classes = np.random.default_rng(5), 6, 2
+    m = Model.create(num_class=classes, max_feature_idx=cols - 1)
+    for i in range(6 * classes):
+        m.add_tree(_tree(rng, int(rng.integers(1, 25)), cols, i == 7))
+    pm = P.parse_model(m.to_text())
+    X = rng.normal(size=(9, cols)).astype(np.float32)
+    for start, num in ((3, 1), (3, 1), (2, 3), (3, 2), (0, 1), (4, 2), (0, -1), (1, 4), (5, 1)):
+        print(f"contrib iterations from {start}, {num}", flush=True)
+        got = be.predict(m, X, "contrib", start_iteration=start, num_iteration=num)
+        ref = np.ascontiguousarray(P.predict_contrib(pm, X, start_iteration=start, num_iteration=num))
+        assert np.array_equal(got.view(np.uint64), ref.view(np.uint64))
