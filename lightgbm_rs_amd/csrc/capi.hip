@@ -36,8 +36,8 @@ void launch_shap_paths(const PredNode* nodes, const PredTree* trees, const doubl
                        const int32_t* cat_bounds, const uint32_t* cat_words,
                        const double* node_cover, const double* leaf_cover, const double* expected,
                        const ShapLeaf* leaves, const ShapStep* steps, const int32_t* feats,
-                       const ShapPlan* plan, int32_t base, int64_t max_items, const float* X,
-                       int64_t rows, int32_t cols, int32_t nf, int32_t max_leaves, int32_t t0, int32_t t1,
+                       const ShapPlan* plan, int64_t max_items, const float* X, int64_t rows,
+                       int32_t cols, int32_t nf, int32_t max_leaves, int32_t t0, int32_t t1,
                        int32_t leaf0, int32_t leaf1, int32_t ntpi, int first, double* tab,
                        double* out, hipStream_t s);
 void launch_csr_dense(const int64_t* indptr, const int32_t* indices, const float* values,
@@ -3486,8 +3486,8 @@ int contrib_paths(lgbm_hip_ctx* c, const lgbm_hip_model* m, const float* d_x, in
       const Run& R = runs[i];
       const PredTree& last = m->tree_index[(size_t)R.t1 - 1];
       launch_shap_paths(c->pm_nodes, c->pm_trees, c->pm_leaves, c->pm_catb, c->pm_catw,
-                        c->pm_ncov, c->pm_lcov, c->pm_expv, c->pm_sleaf, c->pm_sstep,
-                        c->pm_sfeat, c->pm_splan, base, R.items, d_x + r0 * cols,
+                        c->pm_ncov, c->pm_lcov, c->pm_expv, c->pm_sleaf - base, c->pm_sstep,
+                        c->pm_sfeat, c->pm_splan - base, R.items, d_x + r0 * cols,
                         std::min(chunk, rows - r0), cols, nf, max_leaves, R.t0, R.t1,
                         m->tree_index[(size_t)R.t0].leaf0, last.leaf0 + last.num_leaves, ntpi,
                         i == 0, (double*)c->pm_shap, d_out + r0 * width, c->stream);

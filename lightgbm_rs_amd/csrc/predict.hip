@@ -678,15 +678,15 @@ __device__ __forceinline__ void wave_lds_sync() {
 // weights and the one fractions (a bit per element) is the same in all lanes.
 __global__ __launch_bounds__(LGBM_WAVE) void k_shap_items(
     PredModelDev M, ShapModelDev S, const ShapLeaf* __restrict__ leaves,
-    const ShapStep* __restrict__ steps, const ShapPlan* __restrict__ plan, int32_t base,
-    int32_t leaf0, const float* __restrict__ X, int64_t rows, int32_t cols, double* __restrict__ tab) {
+    const ShapStep* __restrict__ steps, const ShapPlan* __restrict__ plan, int32_t leaf0,
+    const float* __restrict__ X, int64_t rows, int32_t cols, double* __restrict__ tab) {
   constexpr int D = SHAP_MAX_DEPTH + 1;
   __shared__ double pw[D][LGBM_WAVE];
   __shared__ double zero[D], ratio[D];
   __shared__ int32_t feat[D];
   const int32_t leaf = leaf0 + (int32_t)blockIdx.x;
-  const ShapLeaf L = leaves[leaf - base];
-  const ShapPlan P = plan[leaf - base];
+  const ShapLeaf L = leaves[leaf];
+  const ShapPlan P = plan[leaf];
   const int32_t depth = L.dm & 0xffff, m = L.dm >> 16;
   const bool by_row = (P.items & SHAP_BY_ROW) != 0u;
   // the plan's row chunk can be larger than the last one
@@ -799,7 +799,7 @@ __host__ __device__ inline size_t shap_row_lds(int32_t nf, int32_t max_leaves) {
 __global__ __launch_bounds__(256) void k_shap_rows(
     PredModelDev M, ShapModelDev S, const ShapLeaf* __restrict__ leaves,
     const ShapStep* __restrict__ steps, const int32_t* __restrict__ feats,
-    const ShapPlan* __restrict__ plan, int32_t base, const double* __restrict__ tab,
+    const ShapPlan* __restrict__ plan, const double* __restrict__ tab,
     const float* __restrict__ X, int64_t rows, int32_t cols, int32_t nf, int32_t max_leaves,
     int32_t t0, int32_t t1, int32_t ntpi, int32_t first, double* __restrict__ out) {
   extern __shared__ __align__(16) char shap_lds[];
@@ -836,8 +836,8 @@ __global__ __launch_bounds__(256) void k_shap_rows(
       }
       wave_lds_sync();
       for (int32_t l = gl; l < nl; l += G) {
-        const ShapLeaf L = leaves[T.leaf0 - base + l];
-        const ShapPlan P = plan[T.leaf0 - base + l];
+        const ShapLeaf L = leaves[T.leaf0 + l];
+        const ShapPlan P = plan[T.leaf0 + l];
         const int32_t depth = L.dm & 0xffff;
         uint32_t hot = 0u, rank = 0u;
         for (int32_t j = 0; j < depth; ++j) {
@@ -889,15 +889,15 @@ int32_t shap_rows_per_block(int32_t nf, int32_t max_leaves) {
   return 0;
 }
 
-// Trees [t0, t1) whose leaves are [leaf0, leaf1), with paths and plan from leaf `base` on,
-// over rows [0, rows) of X: their values into `tab`, then the rows' sums (continued from
-// `out` unless `first`).
+// Trees [t0, t1) whose leaves are [leaf0, leaf1), over rows [0, rows) of X: their values
+// into `tab`, then the rows' sums (continued from `out` unless `first`).  `leaves` and `plan`
+// are indexed by a leaf's number in the model; only those leaves' are read.
 void launch_shap_paths(const PredNode* nodes, const PredTree* trees, const double* leaf_values,
                        const int32_t* cat_bounds, const uint32_t* cat_words,
                        const double* node_cover, const double* leaf_cover, const double* expected,
                        const ShapLeaf* leaves, const ShapStep* steps, const int32_t* feats,
-                       const ShapPlan* plan, int32_t base, int64_t max_items, const float* X,
-                       int64_t rows, int32_t cols, int32_t nf, int32_t max_leaves, int32_t t0, int32_t t1,
+                       const ShapPlan* plan, int64_t max_items, const float* X, int64_t rows,
+                       int32_t cols, int32_t nf, int32_t max_leaves, int32_t t0, int32_t t1,
                        int32_t leaf0, int32_t leaf1, int32_t ntpi, int first, double* tab,
                        double* out, hipStream_t s) {
   const PredModelDev M{nodes, trees, leaf_values, cat_bounds, cat_words, nullptr, nullptr, nullptr};
@@ -905,11 +905,11 @@ void launch_shap_paths(const PredNode* nodes, const PredTree* trees, const doubl
   // a few waves share a leaf's items where they are many
   const int64_t gy = std::min<int64_t>(std::max<int64_t>((max_items + 255) / 256, 1), 64);
   k_shap_items<<<dim3((unsigned)(leaf1 - leaf0), (unsigned)gy), dim3(LGBM_WAVE), 0, s>>>(
-      M, S, leaves, steps, plan, base, leaf0, X, rows, cols, tab);
+      M, S, leaves, steps, plan, leaf0, X, rows, cols, tab);
   const int32_t rpb = shap_rows_per_block(nf, max_leaves);
   k_shap_rows<<<dim3((unsigned)((rows + rpb - 1) / rpb)), dim3(rpb * SHAP_LANES),
                 shap_row_lds(nf, max_leaves) * (size_t)rpb, s>>>(
-      M, S, leaves, steps, feats, plan, base, tab, X, rows, cols, nf, max_leaves, t0, t1, ntpi, first, out);
+      M, S, leaves, steps, feats, plan, tab, X, rows, cols, nf, max_leaves, t0, t1, ntpi, first, out);
 }
 
 // Path elements and stack entries one thread needs for trees of depth at most `depth`.
