@@ -3499,11 +3499,12 @@ int contrib_paths(lgbm_hip_ctx* c, const lgbm_hip_model* m, const float* d_x, in
 
 // The call as predict_lds_shape sees it: rows of `cols` columns in memory.
 PredCall predict_call(const lgbm_hip_ctx* c, const lgbm_hip_model* m, int64_t rows, int32_t cols,
-                      int32_t it0, int32_t it1, PredForm form, int64_t nnz = 0) {
+                      int32_t it0, int32_t it1, int32_t kind, PredForm form, int64_t nnz = 0) {
   return PredCall{rows, cols, c->pack.stride,
                   (it1 - it0) * m->num_tree_per_iteration,
                   (double)m->leaf_values.size() / (double)std::max<size_t>(m->tree_index.size(), 1),
-                  form, (double)nnz / (double)std::max<int64_t>(rows, 1)};
+                  form, (double)nnz / (double)std::max<int64_t>(rows, 1),
+                  kind == LGBM_HIP_PREDICT_TRANSFORMED ? m->num_tree_per_iteration : 0};
 }
 
 // Enqueues k_predict_lds over R's rows.
@@ -3569,7 +3570,7 @@ int predict_run(lgbm_hip_ctx* c, const lgbm_hip_model* m, const float* d_x, int6
   const PredShape shape =
       es_freq > 0 || !c->pack.words
           ? PredShape{0, 0, 0}
-          : predict_lds_shape(predict_call(c, m, rows, cols, it0, it1, form));
+          : predict_lds_shape(predict_call(c, m, rows, cols, it0, it1, kind, form));
   if (shape.rb > 0) {
     PredRows R{};
     R.dense = d_x;
@@ -3676,7 +3677,7 @@ int predict_sparse(lgbm_hip_ctx* c, const lgbm_hip_model* m, const int64_t* indp
   const PredShape shape =
       csc || kind == LGBM_HIP_PREDICT_CONTRIB || !c->pack.words
           ? PredShape{0, 0, 0}
-          : predict_lds_shape(predict_call(c, m, num_rows, fw, it0, it1, PRED_CSR, nnz));
+          : predict_lds_shape(predict_call(c, m, num_rows, fw, it0, it1, kind, PRED_CSR, nnz));
   const bool direct = shape.rb > 0;
   const size_t xb = direct ? 0 : (size_t)num_rows * (size_t)std::max(fw, 1) * 4;
   const size_t ob = (size_t)num_rows * (size_t)width * (kind == LGBM_HIP_PREDICT_LEAF ? 4 : 8);

@@ -29,12 +29,13 @@ struct PredCall {
   double leaves;       // of a tree on average
   PredForm form;
   double entries;      // PRED_CSR: of a row on average
+  int32_t transformed; // outputs of a row that ConvertOutput reads again, 0 if it has no call
 };
 
 // Times of the two kernels in microseconds, a launch included; the larger term of each line
 // is what bounds it.  The constants are fits to 828 dense calls (64 to 1M rows x 12 to 3900
 // columns, 1 to 300 trees of 15 to 900 leaves): the kernel that the sums name took at most
-// 1.1 times the other's time and a microsecond more, in all but one (1.14 times).
+// 1.1 times the other's time and a microsecond more, in all but 2 (1.14 and 1.21 times).
 inline double predict_time(const PredCall& c) {
   const bool sparse = c.form != PRED_DENSE, staged = c.width <= PRED_STAGE_COLS;
   // rows of mostly zeros take the same shorter walks
@@ -54,8 +55,10 @@ inline double predict_lds_time(const PredCall& c, const PredShape& s) {
   const double rounds = (double)(((c.rows + s.rb - 1) / s.rb + PRED_FILL - 1) / PRED_FILL);
   const int32_t groups = PRED_THREADS / s.rb;
   const double batches = (c.n_trees + s.nb - 1) / s.nb, side = (s.nb + groups - 1) / groups;
+  // a block of all its threads a CU has no other to go on beside its rows' transform
+  const double transform = groups == 1 && c.transformed > 1 ? 1.1e-5 * (double)c.rows * c.transformed : 0.0;
   // the rows' staging: latency, or the memory's rate; then a batch's load and its walks
-  return 15.0 + std::max(rounds * s.rb * c.width / 8192.0, (double)c.rows * c.width * 4.0 / 3.7e6) +
+  return 15.0 + transform + std::max(rounds * s.rb * c.width / 8192.0, (double)c.rows * c.width * 4.0 / 3.7e6) +
          rounds * batches * (0.8 + 0.2 * side * std::log2(std::max(c.leaves, 2.0)));
 }
 
@@ -69,7 +72,8 @@ inline double predict_lds_time(const PredCall& c, const PredShape& s) {
 // and k_predict_lds 1 tree 32 and 231 us, 10 trees 195 and 241, 30 trees 540 and 290.  And
 // wide rows leave LDS for few large trees, so that a block's walks are few: 200k rows x 3900
 // columns, 300 trees of 255 leaves 9.8 and 30.4 ms (2000 columns 9.1 and 14.3, 1000 columns
-// 8.4 and 7.3).
+// 8.4 and 7.3).  One iteration of many classes, transformed, is k_predict's on many narrow
+// rows: 600k x 28, 60 classes 1.74 and 2.08 ms (ten iterations 5.8 and 5.4).
 inline PredShape predict_lds_shape(const PredCall& c) {
   PredShape best{0, 0, 0};
   if (c.n_trees < 1 || c.width < 1 || c.tree_words > PRED_TREE_WORDS) return best;
@@ -91,7 +95,7 @@ inline PredShape predict_lds_shape(const PredCall& c) {
   // made dense first: the dense rows' write, or a thread a row that takes its entries in turn
   const double dense = c.form != PRED_CSR ? 0.0 : 15.0 +
       std::max((double)c.rows * c.width * 4.0 / 3.2e6, 1.15 * c.entries);
-  if (predict_lds_time(c, best) > 1.05 * (predict_time(c) + dense)) return PredShape{0, 0, 0};
+  if (predict_lds_time(c, best) > 1.05 * (predict_time(c) + dense) - 1.0) return PredShape{0, 0, 0};
   return best;
 }
 

@@ -13,9 +13,9 @@ SRC = r"""
 #include <cstdio>
 #include "predict_shape.h"
 int main() {
-  long long rows; int width, words, trees, form; double leaves, entries;
-  while (std::scanf("%lld %d %d %d %lf %d %lf", &rows, &width, &words, &trees, &leaves, &form, &entries) == 7) {
-    const lgbm::PredShape s = lgbm::predict_lds_shape({rows, width, words, trees, leaves, (lgbm::PredForm)form, entries});
+  long long rows; int width, words, trees, form, transformed; double leaves, entries;
+  while (std::scanf("%lld %d %d %d %lf %d %lf %d", &rows, &width, &words, &trees, &leaves, &form, &entries, &transformed) == 8) {
+    const lgbm::PredShape s = lgbm::predict_lds_shape({rows, width, words, trees, leaves, (lgbm::PredForm)form, entries, transformed});
     std::printf("%d %d %zu\n", s.rb, s.nb, s.lds);
   }
 }
@@ -37,8 +37,8 @@ def shape(tmp_path_factory):
     return run
 
 
-def _call(rows, cols, leaves, trees, form=0, entries=0):
-    return (rows, cols, 3 * leaves - 1, trees, leaves, form, entries)
+def _call(rows, cols, leaves, trees, form=0, entries=0, transformed=0):
+    return (rows, cols, 3 * leaves - 1, trees, leaves, form, entries, transformed)
 
 
 def test_blocks_fit_the_kernel(shape):
@@ -47,7 +47,7 @@ def test_blocks_fit_the_kernel(shape):
         (1, 2, 31, 700, 1365, 1366), (0, 1, 3, 100, 20000), (0, 1, 2))]
     taken = 0
     for c, (rb, nb, lds) in zip(calls, shape(calls)):
-        rows, width, words, trees, _, _, _ = c
+        rows, width, words, trees, *_ = c
         if rb == 0:
             continue
         taken += 1
@@ -66,7 +66,7 @@ def test_what_does_not_fit_is_refused(shape):
         _call(100, 0, 31, 50)]))
 
 
-# (rows, columns, leaves, trees, CSR, entries a row): k_predict and k_predict_lds, us
+# (rows, columns, leaves, trees, CSR, entries a row, outputs transformed): k_predict and k_predict_lds, us
 @pytest.mark.parametrize("call,walk,lds", [
     ((200000, 120, 31, 1), 27, 46), ((200000, 500, 31, 1), 31, 134), ((200000, 500, 31, 3), 59, 127),
     ((200000, 1000, 31, 3), 66, 229), ((200000, 1000, 31, 10), 195, 241), ((200000, 3900, 31, 1), 33, 840),
@@ -79,14 +79,16 @@ def test_what_does_not_fit_is_refused(shape):
     ((200000, 500, 255, 30), 809, 469), ((20000, 1000, 31, 10), 69, 39), ((200000, 1000, 31, 30), 540, 290),
     ((20000, 2000, 255, 30), 276, 192), ((200000, 3900, 31, 300), 5849, 3923),
     ((250000, 500, 31, 1, 1, 10), 179, 149), ((2000, 3900, 31, 1, 1, 78), 98, 14),
-    ((250000, 60, 255, 100, 1, 1.2), 665, 294), ((60000, 500, 31, 1, 1, 50), 128, 59)])
+    ((250000, 60, 255, 100, 1, 1.2), 665, 294), ((60000, 500, 31, 1, 1, 50), 128, 59), ((600000, 28, 31, 60, 0, 0, 60), 1741, 2078),
+    ((600000, 28, 31, 60), 755, 513), ((600000, 28, 31, 600, 0, 0, 60), 5785, 5372),
+    ((600000, 200, 31, 60, 0, 0, 60), 4744, 1341), ((100000, 28, 31, 1), 19, 21)])
 def test_measured_calls_take_the_faster_kernel(shape, call, walk, lds):
     assert (shape([_call(*call)])[0][0] > 0) == (lds < walk)
 
 
 def test_a_call_left_to_k_predict_stays_there(shape):
     """Rows made dense for k_predict are not given to k_predict_lds after all."""
-    calls = [c[:-2] for c in (_call(*c) for c in itertools.product(
+    calls = [c[:-3] for c in (_call(*c) for c in itertools.product(
         (64, 8000, 60000, 200000), (12, 63, 64, 350, 2000, 4000), (15, 63, 255, 900), (1, 5, 20, 200)))]
-    csr, made = shape([c + (1, 0.05 * c[1]) for c in calls]), shape([c + (2, 0) for c in calls])
+    csr, made = shape([c + (1, 0.05 * c[1], 0) for c in calls]), shape([c + (2, 0, 0) for c in calls])
     assert all(b[0] == 0 for a, b in zip(csr, made) if a[0] == 0)
