@@ -641,7 +641,7 @@ def main():
             "binning": _line("k_bin_records (ValueToBin + record packing, f32 column-major "
                              "input)", bin_tm["bin_ms"], bin_tm["bin_launches"],
                              n * (28 * 4 + int(rec)), f"{n} rows x 28 features"),
-            "predict": _line("k_predict (raw scores)", pred_tm["predict_ms"],
+            "predict": _line("k_predict_lds (raw scores)", pred_tm["predict_ms"],
                              pred_tm["predict_launches"], pred_rows * (28 * 4 + 8),
                              f"{pred_rows} rows x {len(trees)} trees of {nl} leaves",
                              walks=pred_tm["predict_walks"]),

@@ -1,12 +1,16 @@
-// predict.hip — batch prediction of a LightGBM model over dense f32 rows.
+// predict.hip — batch prediction of a LightGBM model over f32 rows, dense or CSR.
 //
-// One thread per row walks every tree of the requested iteration range on the raw
-// feature values (no binning), as the reference predictor does:
+// A row walks every tree of the requested iteration range on its raw feature values (no
+// binning), as the reference predictor does:
 //   Tree::get_leaf / numerical_decision / categorical_decision (tree.rs:160-340),
 //   GbdtModel::predict_raw (ensemble.rs:75-102): per class an f64 sum over the
-//   iterations in order, starting from 0.0 — here class by class, which adds each
-//   class's trees in the same order,
+//   iterations in order, starting from 0.0 — here each class's trees are added in that
+//   order, whichever class comes first,
 //   ConvertOutput (objective.rs:241-340) for the transformed kind.
+// k_predict_lds walks trees from LDS, several of a row side by side; k_predict, a thread a
+// row, has what that does not take and the calls where it is the faster (predict_shape.h).
+// Feature contributions (TreeSHAP) go by leaf paths (k_shap_items, k_shap_rows) or, past
+// their limits, a thread a row (k_contrib).
 #include <hip/hip_runtime.h>
 
 #include "kernels.h"
