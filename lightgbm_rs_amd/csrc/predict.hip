@@ -227,7 +227,7 @@ __global__ __launch_bounds__(256) void k_predict(PredModelDev M, const float* __
 // The usual prediction (no early stop, constant leaves, trees that fit): a block stages
 // `rb` rows and walks the trees, a few at a time, from LDS too.  A node is one 8-byte
 // word pair (model.h) and its children are neighbours, so a step is two LDS reads (the
-// node, the row's value) and ten VALU instructions, where k_predict gathers 24 bytes a
+// node, the row's value) and 15 VALU instructions, where k_predict gathers 24 bytes a
 // node from L2.  Thresholds are f32: for an f32 value v, v <= thr exactly when v <= the
 // largest float not above thr.
 //
@@ -238,8 +238,9 @@ __global__ __launch_bounds__(256) void k_predict(PredModelDev M, const float* __
 // while the next batch is walked.
 //
 // Measured against k_predict: 2M rows x 28 columns, 100 trees of 255 leaves 3.31 -> 1.53
-// ms, now bound by the bank conflicts of the two gathers (27 LDS cycles a wave and step);
-// 64 rows, 100 trees of 31 leaves 273 -> 14 us (one thread walked all trees); 200003 CSR
+// ms, now bound by the chain of a walk's reads, which four waves a SIMD do not cover (of the
+// CUs' busy cycles VALU 67 %, LDS 35 %, four tenths of it conflicts; waves wait 59 % of
+// theirs); 64 rows, 100 trees of 31 leaves 273 -> 14 us (one thread walked all trees); 200003 CSR
 // rows x 500 columns, 200 trees of 63 leaves 3.84 (with the densify) -> 1.00 ms.  Blocks
 // of half the LDS, two a CU, took 2.55 ms on the first and 2.10 on the third.
 constexpr int32_t PRED_WORDS = PRED_TREE_WORDS / PRED_THREADS;  // a thread stages of a batch
@@ -667,7 +668,8 @@ __global__ __launch_bounds__(256) void k_contrib(PredModelDev M, ShapModelDev S,
 // 50000 rows x 100 trees of 31 leaves (28 features): the one-thread-per-row kernel
 // (k_contrib, kept for deeper and wider trees) took 201.5 ms, bound by its path buffers
 // in memory, 28 bytes an element and quadratic in the depth.  Here the values take 0.10
-// ms and the sums 2.47 ms, bound by the latency of the gathers per leaf.
+// ms and the sums 2.45 ms, bound by the latency of the gathers per leaf (waves wait 71 % of
+// their cycles) and by LDS (57 % of the CUs' busy cycles, seven tenths of it conflicts).
 constexpr int32_t SHAP_LANES = 8;  // lanes a row: unique paths are mostly this short
 constexpr size_t SHAP_LDS = 64 * 1024;
 
