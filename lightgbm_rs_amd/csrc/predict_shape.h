@@ -29,11 +29,10 @@ struct PredCall {
   double leaves;       // of a tree on average
   PredForm form;
   double entries;      // PRED_CSR: of a row on average
-  int32_t transformed; // outputs of a row that ConvertOutput reads again, 0 if it has no call
+  int32_t transformed; // outputs of a row that ConvertOutput goes over again, or 0
 };
 
-// Times of the two kernels in microseconds, a launch included; the larger term of each line
-// is what bounds it.  The constants are fits to 828 dense calls (64 to 1M rows x 12 to 3900
+// Times of the two kernels in microseconds, a launch included.  The constants are fits to 828 dense calls (64 to 1M rows x 12 to 3900
 // columns, 1 to 300 trees of 15 to 900 leaves): the kernel that the sums name took at most
 // 1.1 times the other's time and a microsecond more, in all but 2 (1.14 and 1.21 times).
 inline double predict_time(const PredCall& c) {
@@ -55,10 +54,14 @@ inline double predict_lds_time(const PredCall& c, const PredShape& s) {
   const double rounds = (double)(((c.rows + s.rb - 1) / s.rb + PRED_FILL - 1) / PRED_FILL);
   const int32_t groups = PRED_THREADS / s.rb;
   const double batches = (c.n_trees + s.nb - 1) / s.nb, side = (s.nb + groups - 1) / groups;
-  // a block of all its threads a CU has no other to go on beside its rows' transform
-  const double transform = groups == 1 && c.transformed > 1 ? 1.1e-5 * (double)c.rows * c.transformed : 0.0;
-  // the rows' staging: latency, or the memory's rate; then a batch's load and its walks
-  return 15.0 + transform + std::max(rounds * s.rb * c.width / 8192.0, (double)c.rows * c.width * 4.0 / 3.7e6) +
+  // the rows' staging: latency, or the memory's rate
+  const double stage = std::max(rounds * s.rb * c.width / 8192.0,
+                                (double)c.rows * c.width * 4.0 / 3.7e6);
+  // where each thread has a row, no other block of the CU goes on beside the rows' transform
+  const double transform =
+      groups == 1 && c.transformed > 1 ? 1.1e-5 * (double)c.rows * c.transformed : 0.0;
+  // and a batch's load and its walks
+  return 15.0 + stage + transform +
          rounds * batches * (0.8 + 0.2 * side * std::log2(std::max(c.leaves, 2.0)));
 }
 
